@@ -558,7 +558,10 @@ class Model:
         Explanations and, with use_gpu=True (the default on this device
         path), margins and values run on the GPU (`device`, default the
         training device); use_gpu=False scores margins and values on the
-        host. Every result equals the reference CPU engine's bit for bit.
+        host. Margins, values, leaf ids and Saabas attributions equal the
+        reference CPU engine's bit for bit; TreeSHAP contributions and
+        interactions of trees of at most 8 levels are sums in another order,
+        closer to exact arithmetic (within 1e-5 of the engine's).
         """
         del header, predict_threads  # file inputs and CPU worker counts do not apply
         if isinstance(data, (str, bytes)) or hasattr(data, "__fspath__") or (

@@ -572,4 +572,53 @@ constexpr uint32_t MAX_DEVICE_CATS = 4096;
 // Distinct split features of one tree the TreeSHAP kernel accepts.
 constexpr uint32_t MAX_SHAP_UNIQUE = 1024;
 
+// ---- TreeSHAP of trees of at most SHAP_PATHS_DEPTH split levels
+// (fbhip_shap_paths.hip).
+constexpr int SHAP_PATHS_DEPTH = 8;
+constexpr uint32_t SHAP_PATHS_CHUNKS = 8;    // runs of trees summed by waves of their own
+constexpr uint32_t SHAP_PATHS_PITCH = 65;    // floats between two features' sums of 64 rows
+constexpr uint32_t SHAP_PATHS_MAX_F = 600;   // features whose sums and cells of 64 rows fit LDS
+
+// A split node in its tree's preorder (split nodes only).
+struct PathNodeDev {
+    // PATH_LEAF_L / _R, PATH_AGAIN, the older occurrence's depth << PATH_OLDER,
+    // << PATH_PARTNERS the depths of the path that hold another feature's
+    // newest split, and << PATH_FEATURE the feature
+    uint32_t meta;
+    float al, ar;       // 1 / z - 1 of the left and right edge, z over the feature's path splits
+    float vl, vr;       // a leaf child's value times its path's weights; 0 for a split child
+    float s0;           // vl + vr
+    uint32_t pad[2];
+};
+constexpr uint32_t PATH_LEAF_L = 1u, PATH_LEAF_R = 2u;
+constexpr uint32_t PATH_AGAIN = 4u;  // the feature is on the path above
+constexpr uint32_t PATH_OLDER = 3, PATH_PARTNERS = 8, PATH_FEATURE = 16;
+
+// The same node's test.
+struct PathTestDev {
+    uint32_t ff;        // feature | PATH_DEFAULT_LEFT | PATH_CAT
+    float cond;
+    uint32_t cat_offset, cat_len;
+};
+constexpr uint32_t PATH_DEFAULT_LEFT = 1u << 30, PATH_CAT = 1u << 29, PATH_FEAT = PATH_CAT - 1;
+
+struct ShapPaths {
+    const PathNodeDev *nodes;  // one more than the split nodes
+    const PathTestDev *tests;
+    const uint32_t *first;     // [n_trees + 1] first split node of a tree
+    const uint32_t *cats;
+    uint32_t n_trees, n_features;
+    uint32_t stride;           // masks of a tree: more than its split nodes
+    uint32_t run_trees, runs;  // trees a wave walks, and runs of them
+    float bias, root_mean;
+};
+// Device bytes launch_shap_paths needs for 64 rows.
+uint64_t shap_paths_tile_bytes(const ShapPaths &m, bool inter);
+// Contributions (out [n_rows][n_features + 1]) or interactions (out
+// [n_rows][n_features + 1][n_features + 1]) of device rows, through `work`
+// (at least 64 rows' bytes; the more it holds, the more rows run at once).
+hipError_t launch_shap_paths(const ShapPaths &m, bool inter, const float *rows, uint64_t n_rows,
+                             const float *margin, float *out, void *work, uint64_t work_bytes,
+                             hipStream_t s);
+
 }  // namespace fbh

@@ -784,11 +784,17 @@ struct fbh_shap_model {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     double last_ms = 0.0;
     std::vector<void *> allocs;
+    ShapPaths paths{};        // fbhip_shap_paths.hip; nodes null where the trees do not fit it
+    bool host_order = false;  // fbh_shap_set_host_order
+    void *work = nullptr;     // launch_shap_paths's workspace, kept between calls
+    uint64_t work_bytes = 0;
+    std::mutex work_mu;       // held while the kernels that share it are enqueued
 
     ~fbh_shap_model() {
         if (device >= 0) (void)hipSetDevice(device);
         if (stream) (void)hipStreamSynchronize(stream);
         for (void *p : allocs) (void)hipFree(p);
+        if (work) (void)hipFree(work);
         if (e0) (void)hipEventDestroy(e0);
         if (e1) (void)hipEventDestroy(e1);
         if (stream) (void)hipStreamDestroy(stream);
@@ -851,6 +857,126 @@ float node_means(const std::vector<int32_t> &left, const std::vector<int32_t> &r
     }
     means[g] = value;
     return value;
+}
+
+// The split nodes of a tree in preorder as fbhip_shap_paths.hip walks them; false
+// where its arithmetic would leave the range of a float (covers or leaf values
+// near its limits) or a threshold is NaN.
+struct PathBuild {
+    std::vector<PathNodeDev> nodes;
+    std::vector<PathTestDev> tests;
+    std::vector<uint32_t> first{0};
+    bool ok = true;
+
+    void add_tree(const std::vector<ShapNodeDev> &n, uint32_t root) {
+        std::vector<Edge> path;
+        if (ok && !(n[root].flags & 1u)) add(n, root, path, 1.0);
+        first.push_back((uint32_t)nodes.size());
+    }
+
+private:
+    // an edge of the path: its feature, and the product of the weights of that
+    // feature's edges down to it
+    struct Edge {
+        uint32_t feat;
+        double z;
+    };
+
+    void add(const std::vector<ShapNodeDev> &n, uint32_t id, std::vector<Edge> &path, double weight) {
+        const ShapNodeDev &d = n[id];
+        const int depth = (int)path.size();
+        if (depth >= SHAP_PATHS_DEPTH) ok = false;
+        if (!ok) return;
+        PathNodeDev p{};
+        PathTestDev t{};
+        t.ff = d.feat | ((d.flags & 2u) ? PATH_DEFAULT_LEFT : 0u) | ((d.flags & 4u) ? PATH_CAT : 0u);
+        t.cond = d.split_cond;
+        t.cat_offset = d.cat_offset;
+        t.cat_len = d.cat_len;
+        if (!(d.flags & 4u) && std::isnan(d.split_cond)) ok = false;
+        p.meta = d.feat << PATH_FEATURE;
+        double older = 1.0;
+        for (int k = depth - 1; k >= 0; k--) {
+            if (path[k].feat == d.feat) {
+                if (!(p.meta & PATH_AGAIN)) {
+                    p.meta |= PATH_AGAIN | (uint32_t)k << PATH_OLDER;
+                    older = path[k].z;
+                }
+                continue;
+            }
+            bool newest = true;
+            for (int j = k + 1; j < depth; j++) newest &= path[j].feat != path[k].feat;
+            if (newest) p.meta |= 1u << (PATH_PARTNERS + k);
+        }
+        const uint32_t child[2] = {(uint32_t)d.left, (uint32_t)d.right};
+        const double w[2] = {(double)d.left_weight, (double)d.right_weight};
+        float a[2], v[2] = {0.0f, 0.0f};
+        for (int s = 0; s < 2; s++) {
+            const double hot = 1.0 / (older * w[s]) - 1.0;
+            a[s] = (float)hot;
+            if (!(hot > -1.0 && hot < 1e30)) ok = false;
+            const ShapNodeDev &c = n[child[s]];
+            if (!(c.flags & 1u)) continue;
+            p.meta |= s ? PATH_LEAF_R : PATH_LEAF_L;
+            const double leaf = (double)c.leaf_value * weight * w[s];
+            v[s] = (float)leaf;
+            if (!std::isfinite(leaf) || (leaf != 0.0 && std::fabs(leaf) < 1e-36)) ok = false;
+        }
+        p.al = a[0];
+        p.ar = a[1];
+        p.vl = v[0];
+        p.vr = v[1];
+        p.s0 = v[0] + v[1];
+        nodes.push_back(p);
+        tests.push_back(t);
+        for (int s = 0; s < 2; s++) {
+            if (n[child[s]].flags & 1u) continue;
+            path.push_back({d.feat, older * w[s]});
+            add(n, child[s], path, weight * w[s]);
+            path.pop_back();
+        }
+    }
+};
+
+// Whether launch_shap_paths computes this kind for the model: 64 rows fit the
+// fixed scratch of fbh_shap_contribs_noalloc beside their cells (so that entry
+// gives the same values), and an interaction workspace stays modest.
+bool takes_paths(const fbh_shap_model *m, bool inter) {
+    if (!m->paths.nodes || m->host_order) return false;
+    const uint64_t tile = shap_paths_tile_bytes(m->paths, inter);
+    const uint64_t io = 64ull * 4 * (2ull * m->n_features + 2);
+    return tile <= (inter ? 256ull << 20 : FBH_NOALLOC_SCRATCH_BYTES - 4096 - io);
+}
+
+// Most bytes of a model's kept workspace: 56k rows of 200 features and 100
+// trees of depth 8 at once, which is nine times what fills the device.
+constexpr uint64_t PATHS_WORK_BYTES = 512ull << 20;
+
+// Contributions or interactions by launch_shap_paths through the model's
+// workspace, which grows to what the call can use. Work of earlier calls runs
+// on the same stream before this one's, so it may share the workspace.
+// False (nothing enqueued) when there is no memory for 64 rows.
+bool run_paths(fbh_shap_model *m, bool inter, const float *rows, uint64_t n, const float *margin,
+               float *out) {
+    std::lock_guard<std::mutex> g(m->work_mu);
+    const uint64_t tile = shap_paths_tile_bytes(m->paths, inter);
+    const uint64_t most = std::max<uint64_t>(1, PATHS_WORK_BYTES / tile);
+    const uint64_t want = std::min<uint64_t>((n + 63) / 64, most) * tile;
+    if (m->work_bytes < want) {
+        if (m->work) {
+            chk(hipStreamSynchronize(m->stream), "workspace");
+            chk(hipFree(m->work), "workspace");
+        }
+        m->work = nullptr;
+        m->work_bytes = 0;
+        for (uint64_t b = want; b >= tile && !m->work; b /= 2)
+            if (hipMalloc(&m->work, b) == hipSuccess) m->work_bytes = b;
+            else (void)hipGetLastError();
+        if (!m->work) return false;
+    }
+    chk(launch_shap_paths(m->paths, inter, rows, n, margin, out, m->work, m->work_bytes, m->stream),
+        "shap paths launch");
+    return true;
 }
 
 hipError_t launch_shap(const fbh_shap_model *m, bool inter, const float *rows, uint64_t n_rows,
@@ -925,9 +1051,11 @@ void enqueue(fbh_shap_model *m, Kind k, const float *d_rows, uint64_t n, const f
     const uint32_t blocks = (uint32_t)((n + PRED_TPB - 1) / PRED_TPB);
     switch (k) {
         case Kind::Contribs:
+            if (takes_paths(m, false) && run_paths(m, false, d_rows, n, d_margin, d_out)) return;
             chk(launch_shap(m, false, d_rows, n, d_margin, d_out), "shap launch");
             return;
         case Kind::Interactions:
+            if (takes_paths(m, true) && run_paths(m, true, d_rows, n, d_margin, d_out)) return;
             chk(launch_fill_f32(d_out, 0.0f, n * out_width(m, k), m->stream), "interaction clear");
             chk(launch_shap(m, true, d_rows, n, d_margin, d_out), "interaction launch");
             return;
@@ -971,6 +1099,8 @@ void enqueue(fbh_shap_model *m, Kind k, const float *d_rows, uint64_t n, const f
 struct Staging {
     float *rows = nullptr, *margin = nullptr, *out = nullptr;
     uint64_t cap_rows = 0;
+    void *work = nullptr;  // contributions: launch_shap_paths's workspace, where
+    uint64_t work_bytes = 0;  // the call must not allocate the model's
 };
 
 // Runs one kind over host rows through `st`, batch after batch, and times the
@@ -987,7 +1117,12 @@ void run_host(fbh_shap_model *m, Kind k, const Staging &st, const float *rows, u
             chk(hipMemcpyAsync(st.margin, margin + r0, 4 * b, hipMemcpyHostToDevice, m->stream),
                 "margin upload");
         chk(hipEventRecord(m->e0, m->stream), "event");
-        enqueue(m, k, st.rows, b, margin ? st.margin : nullptr, st.out);
+        if (st.work)
+            chk(launch_shap_paths(m->paths, false, st.rows, b, margin ? st.margin : nullptr, st.out,
+                                  st.work, st.work_bytes, m->stream),
+                "shap paths launch");
+        else
+            enqueue(m, k, st.rows, b, margin ? st.margin : nullptr, st.out);
         chk(hipEventRecord(m->e1, m->stream), "event");
         chk(hipMemcpyAsync(out + r0 * w, st.out, 4 * b * w, hipMemcpyDeviceToHost, m->stream),
             "output download");
@@ -1078,6 +1213,8 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         std::vector<float> means(total, 0.0f);
         std::vector<uint32_t> roots(n_trees), uoff(n_trees + 1, 0), ufeats;
         double rm_sum = 0.0;
+        PathBuild pb;
+        pb.ok = n_features <= SHAP_PATHS_MAX_F;
         for (uint32_t t = 0; t < n_trees; t++) {
             const uint32_t b = tree_offsets[t], e = tree_offsets[t + 1];
             if (e <= b) throw ShapError(FBH_INPUT_ERROR, "tree " + std::to_string(t) + " has no nodes");
@@ -1154,6 +1291,7 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
                 throw ShapError(FBH_INPUT_ERROR, "a tree splits on more than " +
                                                      std::to_string(MAX_SHAP_UNIQUE) +
                                                      " distinct features");
+            pb.add_tree(nodes, b);
             rm_sum += root_mean(L, R, lv, hs, lf, b, 0);
             node_means(L, R, lv, hs, lf, b, 0, means);
         }
@@ -1177,7 +1315,34 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         m->d_ufeats = m->upload(ufeats, "shap features");
         m->d_cats = m->upload(cw, "shap categories");
         m->d_rule = m->upload(rv, "shap rule");
+        if (pb.ok && !pb.nodes.empty() && m->cover_error.empty()) {
+            uint32_t most = 0;
+            for (uint32_t t = 0; t < n_trees; t++) most = std::max(most, pb.first[t + 1] - pb.first[t]);
+            // the walk requests one node past a tree's last, the tests are read
+            // eight at a time
+            pb.nodes.resize(pb.nodes.size() + 1);
+            pb.tests.resize(pb.tests.size() + 8);
+            ShapPaths &q = m->paths;
+            q.tests = m->upload(pb.tests, "path tests");
+            q.first = m->upload(pb.first, "path trees");
+            q.cats = m->d_cats;
+            q.n_trees = n_trees;
+            q.n_features = n_features;
+            q.stride = (most + 8) & ~7u;
+            q.run_trees = (n_trees + SHAP_PATHS_CHUNKS - 1) / SHAP_PATHS_CHUNKS;
+            q.runs = (n_trees + q.run_trees - 1) / q.run_trees;
+            q.bias = bias;
+            q.root_mean = m->root_mean;
+            q.nodes = m->upload(pb.nodes, "path nodes");
+        }
         *out = m.release();
+    });
+}
+
+int fbh_shap_set_host_order(fbh_shap_model *m, int on) {
+    return shap_guard([&] {
+        if (!m) throw ShapError(FBH_INPUT_ERROR, "null argument");
+        m->host_order = on != 0;
     });
 }
 
@@ -1275,12 +1440,24 @@ int fbh_shap_contribs_noalloc(fbh_shap_model *m, const float *rows, uint64_t n_r
         unsigned char *base = static_cast<unsigned char *>(scratch_of(m->device));
         Staging st;
         st.cap_rows = std::min<uint64_t>(cap, n_rows);
+        if (takes_paths(m, false)) {
+            // the rest of the scratch holds the workspace of the same rows
+            const uint64_t tile = shap_paths_tile_bytes(m->paths, false);
+            const uint64_t tiles = std::min<uint64_t>((room - 256) / (64 * per_row + tile),
+                                                      (n_rows + 63) / 64);
+            st.cap_rows = std::min<uint64_t>(tiles * 64, n_rows);
+            st.work_bytes = tiles * tile;
+        }
         st.rows = reinterpret_cast<float *>(base);
         st.margin = reinterpret_cast<float *>(base + round256(4 * st.cap_rows * nf));
         st.out = reinterpret_cast<float *>(reinterpret_cast<unsigned char *>(st.margin) +
                                            round256(4 * st.cap_rows));
-        if ((reinterpret_cast<unsigned char *>(st.out) - base) + 4 * st.cap_rows * w >
-            NOALLOC_SCRATCH_BYTES)
+        unsigned char *end = reinterpret_cast<unsigned char *>(st.out) + 4 * st.cap_rows * w;
+        if (st.work_bytes) {
+            st.work = reinterpret_cast<unsigned char *>(st.out) + round256(4 * st.cap_rows * w);
+            end = static_cast<unsigned char *>(st.work) + st.work_bytes;
+        }
+        if ((uint64_t)(end - base) > NOALLOC_SCRATCH_BYTES)
             throw ShapError(FBH_RUNTIME_ERROR, "fbh_shap_contribs_noalloc: scratch layout overflow");
         run_host(m, Kind::Contribs, st, rows, n_rows, margin, out);
     });

@@ -330,6 +330,11 @@ void sort_row_ascending(float *row, uint32_t k) {
     }
 }
 
+// Explanations of fewer rows of a multi-output model keep the host engine's
+// operation order: small samples are compared with its per-class values bit for
+// bit. Larger ones take the backend's default.
+constexpr uint64_t HOST_ORDER_ROWS = 512;
+
 // A multiclass model's outputs: each class scored or explained by its own
 // trees with its own intercept (Model::class_view, src/model/tree.rs:
 // 395-425), the per-class results laid out [row][class][...].
@@ -367,6 +372,8 @@ void predict_multiclass(const fbt::Model &m, const float *x, uint64_t n_rows, ui
         } else {
             ShapModel sm = explain_model(m, ids, bias, device);
             int rc = FBH_OK;
+            if (!scores && n_rows < HOST_ORDER_ROWS) rc = fbh_shap_set_host_order(sm.get(), 1);
+            if (rc) backend_fail(rc);
             if (scores) rc = fbh_predict(sm.get(), x, n_rows, bm, FBH_PREDICT_MARGIN, col.data());
             else if (output == FBT_OUT_CONTRIBS) rc = fbh_shap_contribs(sm.get(), x, n_rows, bm, col.data());
             else if (output == FBT_OUT_APPROX_CONTRIBS)

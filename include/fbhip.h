@@ -609,6 +609,13 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
                           uint32_t n_cat_words, uint32_t n_features, float bias,
                           fbh_shap_model **out);
 int fbh_shap_model_destroy(fbh_shap_model *m);
+/* Contributions and interactions of trees of at most 8 split levels are taken
+ * by default from closed sums of the same quadrature (no divides; the values of
+ * exact arithmetic to within float rounding, closer than the host engine's
+ * order gives them). on != 0: always the host engine's float operations in its
+ * order, whose results equal the CPU engine's bit for bit. No reference
+ * counterpart. */
+int fbh_shap_set_host_order(fbh_shap_model *m, int on);
 /* GpuExplainModel::compute (src/backend/cuda/explain.rs:491-843) for
  * pred_contribs: rows row-major [n_rows][n_features], optional per-row
  * margin replacing the bias, out [n_rows][n_features + 1]. */
