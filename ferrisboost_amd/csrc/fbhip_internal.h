@@ -621,4 +621,51 @@ hipError_t launch_shap_paths(const ShapPaths &m, bool inter, const float *rows, 
                              const float *margin, float *out, void *work, uint64_t work_bytes,
                              hipStream_t s);
 
+// ---- Prediction with rows and runs of trees in LDS (fbhip_predict.hip).
+// Output kinds of a prediction; PRED_OUT_VALUES: each tree's leaf value,
+// [n_trees][n_rows], for predict_sum_kernel.
+enum { PRED_OUT_MARGIN = 0, PRED_OUT_SIGMOID = 1, PRED_OUT_LEAF = 2, PRED_OUT_VALUES = 3 };
+// A node: x the threshold's key (plus 2 where a missing value goes left), a
+// leaf's value's bits, or a categorical split's set (first word in the run's
+// entries | words << 16); y the left child's entry in the run (the right one
+// follows it; a leaf: its own) << PRED_CHILD, the feature << PRED_FEAT, flags.
+constexpr uint32_t PRED_DL_BIT = 2u, PRED_CHILD = 2, PRED_CHILD_MASK = 0x3FFFu;
+constexpr uint32_t PRED_CAT_BIT = 1u << 16, PRED_FEAT = 17, PRED_FEAT_MASK = 0x3FFFu;
+constexpr uint32_t PRED_LEAF_BIT = 1u << 31;
+constexpr uint32_t PRED_KEY_NAN = 0xFFFFFFFEu;
+constexpr uint32_t PRED_CUS = 256;
+// A run of trees in LDS: beside the rows (at most 64 KiB of cells for two or four
+// groups of 64 rows, else 64 rows) and 8 KiB of leaf values it takes what is left
+// of a CU's 160 KiB, and no more than 12,800 entries (25 complete trees of depth 8)
+// or 32 trees, which the waves of a workgroup walk at once.
+// A run's first PRED_RUN_TREES / 2 entries hold its trees' first entries; the words
+// of a tree's category sets follow its nodes.
+constexpr uint32_t PRED_RUN_NODES = 12800, PRED_RUN_TREES = 32;
+constexpr uint32_t PRED_LDS_BYTES = 160 * 1024, PRED_LEAFV_BYTES = 8 * 1024;
+constexpr uint32_t PRED_TILES_MAX_F = 500;  // features of which 64 rows fit beside 2,500 nodes
+constexpr uint32_t PRED_FILL_TILES = 256;   // workgroups that fill the device
+constexpr uint64_t PRED_WORK_BYTES = 64ull << 20;  // most of a split call's leaf values
+
+struct PredRun {
+    uint32_t tree0, n_trees;
+    uint32_t node0, n_nodes;  // node0 even
+};
+struct PredTrees {
+    const uint2 *nodes;         // run after run; null: the model has a tree larger than a run
+    const PredRun *runs;
+    const uint32_t *ids;        // a node's id in the caller's tree
+    uint32_t categorical;       // some split is
+    uint32_t n_trees, n_runs, n_features;
+    uint32_t groups;            // groups of 64 rows a workgroup can hold: 1, 2 or 4
+    uint32_t most_nodes;        // of a run
+};
+// Device bytes of the leaf values a call of so few rows that its runs are split
+// over workgroups goes through (0: none).
+uint64_t predict_tiles_work(const PredTrees &P, uint64_t n_rows, uint32_t mode);
+// Margins, values (PRED_OUT_SIGMOID) or leaf ids; `work` of
+// predict_tiles_work's bytes, or null.
+hipError_t launch_predict_tiles(const PredTrees &P, const float *rows, uint64_t n_rows,
+                                const float *init, float base, uint32_t mode, float *out,
+                                void *work, hipStream_t s);
+
 }  // namespace fbh

@@ -63,7 +63,8 @@ constexpr uint32_t PN_CAT = 1u << 29;
 constexpr uint32_t PN_FEAT = PN_CAT - 1;
 
 // Output kinds of predict_kernel.
-constexpr uint32_t PRED_MARGIN = 0, PRED_SIGMOID = 1, PRED_LEAF = 2;
+constexpr uint32_t PRED_MARGIN = PRED_OUT_MARGIN, PRED_SIGMOID = PRED_OUT_SIGMOID,
+                   PRED_LEAF = PRED_OUT_LEAF;
 
 // categorical::goes_left (src/data/categorical.rs:334-370): a category in the
 // node's right-going set goes right; negative, non-integral-range and
@@ -149,36 +150,15 @@ __global__ __launch_bounds__(PRED_TPB) void predict_kernel(
     predict_row(nodes, full, cats, roots, n_trees, rows + row * nf, row, init, base, mode, out);
 }
 
-// The same walk with a wave's 64 rows first copied into LDS (coalesced
-// loads; row stride nf | 1, odd, so the 64 lanes' cells of one feature fall
-// in distinct banks): a node's cell is then an LDS read instead of a
-// gather of one cache line a lane from the row-major matrix.
 constexpr uint32_t PRED_LDS_ROWS = 64;
-constexpr uint32_t PRED_LDS_MAX_F = 255;  // 64 rows x 256 floats: 64 KiB of LDS
 
-__global__ __launch_bounds__(PRED_LDS_ROWS) void predict_lds_kernel(
-    const PredNodeDev *__restrict__ nodes, const ShapNodeDev *__restrict__ full,
-    const uint32_t *__restrict__ cats, const uint32_t *__restrict__ roots, uint32_t n_trees,
-    const float *__restrict__ rows, uint64_t n_rows, uint32_t nf, const float *__restrict__ init,
-    float base, uint32_t mode, float *__restrict__ out) {
-    extern __shared__ float xs[];
-    const uint32_t S = nf | 1u;
-    const uint64_t r0 = (uint64_t)blockIdx.x * PRED_LDS_ROWS;
-    const uint32_t nr = (uint32_t)min<uint64_t>(PRED_LDS_ROWS, n_rows - r0);
-    const float *src = rows + r0 * nf;
-    for (uint32_t r = 0; r < nr; r++)
-        for (uint32_t f = threadIdx.x; f < nf; f += PRED_LDS_ROWS) xs[r * S + f] = src[r * nf + f];
-    __syncthreads();
-    if (threadIdx.x >= nr) return;
-    predict_row(nodes, full, cats, roots, n_trees, xs + threadIdx.x * S, r0 + threadIdx.x, init,
-                base, mode, out);
-}
-
-// The LDS rows shared by four waves, which take every fourth tree of a run
-// of PRED_RUN trees and put each row's leaf value in LDS; wave 0 then adds
-// the run's values to the row's margin in tree order (the host's f32
-// additions, so the margins stay bit-identical), and the waves go on to the
-// next run. Four times the waves of predict_lds_kernel on the same rows.
+// The same walk, for models with a tree too large for fbhip_predict.hip, over
+// 64 rows copied into LDS (coalesced loads; row stride nf | 1, odd, so the 64
+// lanes' cells of one feature fall in distinct banks) and shared by four
+// waves, which take every fourth tree of a run of PRED_RUN trees and put each
+// row's leaf value in LDS; wave 0 then adds the run's values to the row's
+// margin in tree order (the host's f32 additions, so the margins stay
+// bit-identical), and the waves go on to the next run.
 constexpr uint32_t PRED_WAVES = 4;
 constexpr uint32_t PRED_RUN = 32;
 constexpr uint32_t PRED_LDS4_MAX_F = 223;  // 64 x 224 + 64 x 32 floats: 64 KiB of LDS
@@ -786,7 +766,8 @@ struct fbh_shap_model {
     std::vector<void *> allocs;
     ShapPaths paths{};        // fbhip_shap_paths.hip; nodes null where the trees do not fit it
     bool host_order = false;  // fbh_shap_set_host_order
-    void *work = nullptr;     // launch_shap_paths's workspace, kept between calls
+    PredTrees pred{};         // fbhip_predict.hip; nodes null where a tree does not fit it
+    void *work = nullptr;     // both files' workspace, kept between calls
     uint64_t work_bytes = 0;
     std::mutex work_mu;       // held while the kernels that share it are enqueued
 
@@ -938,6 +919,113 @@ private:
     }
 };
 
+// The trees as fbhip_predict.hip walks them, renumbered level by level so that a
+// node's children are neighbours; ok is false where one is larger than a run.
+struct PredBuild {
+    static constexpr uint32_t HEAD = PRED_RUN_TREES / 2;
+    std::vector<uint2> nodes;
+    std::vector<PredRun> runs;
+    std::vector<uint32_t> ids;
+    bool ok = true, categorical = false;
+    uint32_t done = 0;  // trees
+    uint32_t groups = 1, cap = 0, trees = PRED_RUN_TREES, most_nodes = 0;
+
+    // The rows a workgroup holds, a run's most entries beside them, and its most
+    // trees such that the runs are of a size.
+    PredBuild(uint32_t nf, const uint32_t *offsets, uint32_t n_trees, const uint32_t *cat_len) {
+        const uint32_t row = 4 * (nf | 1u);
+        groups = 256 * row <= 64 * 1024 ? 4 : 128 * row <= 64 * 1024 ? 2 : 1;
+        const uint32_t cells = 64 * groups * row;
+        if (nf > PRED_TILES_MAX_F || n_trees == 0) {
+            ok = false;
+            return;
+        }
+        cap = std::min((PRED_LDS_BYTES - PRED_LEAFV_BYTES - cells - 64) / 8, PRED_RUN_NODES);
+        uint32_t n_runs = 0, in_run = 0;
+        uint64_t entries = HEAD;
+        for (uint32_t t = 0; t < n_trees; t++) {
+            uint64_t words = 0;
+            for (uint32_t i = offsets[t]; cat_len && i < offsets[t + 1]; i++) words += cat_len[i];
+            const uint64_t size = offsets[t + 1] - offsets[t] + (words + 1) / 2;
+            if (n_runs == 0 || in_run == PRED_RUN_TREES || entries + size > cap) {
+                n_runs++;
+                in_run = 0;
+                entries = HEAD;
+            }
+            in_run++;
+            entries += size;
+        }
+        trees = (n_trees + n_runs - 1) / n_runs;
+    }
+
+    static uint32_t key_of(float v) {
+        uint32_t u;
+        v += 0.0f;
+        std::memcpy(&u, &v, 4);
+        return u ^ ((u >> 31) ? 0xFFFFFFFFu : 0x80000000u);
+    }
+
+    void add_tree(const std::vector<ShapNodeDev> &n, uint32_t root, uint32_t count,
+                  const uint32_t *cat_words) {
+        if (!ok) return;
+        std::vector<uint32_t> order{root};
+        uint64_t words = 0;
+        for (uint32_t i = 0; i < order.size() && order.size() <= count; i++) {
+            const ShapNodeDev &d = n[order[i]];
+            if (d.flags & 1u) continue;
+            words += d.cat_len;
+            order.push_back((uint32_t)d.left);
+            order.push_back((uint32_t)d.right);
+        }
+        const uint64_t size = order.size() + (words + 1) / 2;
+        if (order.size() > count || HEAD + size > cap) {  // a node under two parents, or too large
+            ok = false;
+            return;
+        }
+        if (runs.empty() || runs.back().n_trees == trees || runs.back().n_nodes + size > cap) {
+            if (nodes.size() & 1) nodes.push_back(make_uint2(0, 0));  // loaded two at a time
+            runs.push_back({done, 0, (uint32_t)nodes.size(), HEAD});
+            nodes.resize(nodes.size() + HEAD);
+        }
+        PredRun &run = runs.back();
+        uint2 &first = nodes[run.node0 + run.n_trees / 2];
+        (run.n_trees & 1 ? first.y : first.x) = run.n_nodes;
+        done++;
+        ids.resize(nodes.size());
+        std::vector<uint32_t> set;
+        uint32_t child = 1;
+        for (uint32_t i = 0; i < order.size(); i++) {
+            const ShapNodeDev &d = n[order[i]];
+            uint2 p;
+            if (d.flags & 1u) {
+                std::memcpy(&p.x, &d.leaf_value, 4);
+                p.y = (run.n_nodes + i) << PRED_CHILD | PRED_LEAF_BIT;
+            } else {
+                const uint32_t dl = (d.flags & 2u) ? PRED_DL_BIT : 0u;
+                p.y = (run.n_nodes + child) << PRED_CHILD | d.feat << PRED_FEAT | dl;
+                // a NaN threshold: right, but for a missing value
+                p.x = (std::isnan(d.split_cond) ? 0u : key_of(d.split_cond)) + dl;
+                if (d.flags & 4u) {
+                    categorical = true;
+                    p.y |= PRED_CAT_BIT;
+                    p.x = (2 * (run.n_nodes + (uint32_t)order.size()) + (uint32_t)set.size()) |
+                          d.cat_len << 16;
+                    set.insert(set.end(), cat_words + d.cat_offset,
+                               cat_words + d.cat_offset + d.cat_len);
+                }
+                child += 2;
+            }
+            nodes.push_back(p);
+            ids.push_back(order[i] - root);
+        }
+        for (size_t k = 0; k < set.size(); k += 2)
+            nodes.push_back(make_uint2(set[k], k + 1 < set.size() ? set[k + 1] : 0u));
+        run.n_trees++;
+        run.n_nodes += (uint32_t)size;
+        most_nodes = std::max(most_nodes, run.n_nodes);
+    }
+};
+
 // Whether launch_shap_paths computes this kind for the model: 64 rows fit the
 // fixed scratch of fbh_shap_contribs_noalloc beside their cells (so that entry
 // gives the same values), and an interaction workspace stays modest.
@@ -952,28 +1040,44 @@ bool takes_paths(const fbh_shap_model *m, bool inter) {
 // trees of depth 8 at once, which is nine times what fills the device.
 constexpr uint64_t PATHS_WORK_BYTES = 512ull << 20;
 
+// Grows the model's workspace to `want` bytes, or to as much as there is, not
+// below `least`; work_mu must be held. Work of earlier calls runs on the same
+// stream before this one's, so calls share the workspace.
+bool grow_work(fbh_shap_model *m, uint64_t want, uint64_t least) {
+    if (m->work_bytes >= want) return true;
+    if (m->work) {
+        chk(hipStreamSynchronize(m->stream), "workspace");
+        chk(hipFree(m->work), "workspace");
+    }
+    m->work = nullptr;
+    m->work_bytes = 0;
+    for (uint64_t b = want; b >= least && !m->work; b /= 2)
+        if (hipMalloc(&m->work, b) == hipSuccess) m->work_bytes = b;
+        else (void)hipGetLastError();
+    return m->work != nullptr;
+}
+
+// Margins, values or leaf ids by launch_predict_tiles.
+void run_predict(fbh_shap_model *m, const float *rows, uint64_t n, const float *margin,
+                 uint32_t mode, float *out) {
+    const uint64_t bytes = predict_tiles_work(m->pred, n, mode);
+    std::unique_lock<std::mutex> g(m->work_mu, std::defer_lock);
+    if (bytes) g.lock();
+    const bool work = bytes && grow_work(m, bytes, bytes);
+    chk(launch_predict_tiles(m->pred, rows, n, margin, m->bias, mode, out, work ? m->work : nullptr,
+                             m->stream),
+        "predict launch");
+}
+
 // Contributions or interactions by launch_shap_paths through the model's
-// workspace, which grows to what the call can use. Work of earlier calls runs
-// on the same stream before this one's, so it may share the workspace.
-// False (nothing enqueued) when there is no memory for 64 rows.
+// workspace, which grows to what the call can use. False (nothing enqueued) when there is no memory for 64 rows.
 bool run_paths(fbh_shap_model *m, bool inter, const float *rows, uint64_t n, const float *margin,
                float *out) {
     std::lock_guard<std::mutex> g(m->work_mu);
     const uint64_t tile = shap_paths_tile_bytes(m->paths, inter);
     const uint64_t most = std::max<uint64_t>(1, PATHS_WORK_BYTES / tile);
     const uint64_t want = std::min<uint64_t>((n + 63) / 64, most) * tile;
-    if (m->work_bytes < want) {
-        if (m->work) {
-            chk(hipStreamSynchronize(m->stream), "workspace");
-            chk(hipFree(m->work), "workspace");
-        }
-        m->work = nullptr;
-        m->work_bytes = 0;
-        for (uint64_t b = want; b >= tile && !m->work; b /= 2)
-            if (hipMalloc(&m->work, b) == hipSuccess) m->work_bytes = b;
-            else (void)hipGetLastError();
-        if (!m->work) return false;
-    }
+    if (!grow_work(m, want, tile)) return false;
     chk(launch_shap_paths(m->paths, inter, rows, n, margin, out, m->work, m->work_bytes, m->stream),
         "shap paths launch");
     return true;
@@ -1069,20 +1173,16 @@ void enqueue(fbh_shap_model *m, Kind k, const float *d_rows, uint64_t n, const f
             const uint32_t mode = k == Kind::Leaf ? PRED_LEAF
                                   : k == Kind::Value ? PRED_SIGMOID : PRED_MARGIN;
             const uint32_t nf = m->n_features;
-            const char *kind_env = std::getenv("FB_HIP_PREDICT_KERNEL");
-            const int pk = kind_env ? std::atoi(kind_env) : 4;
-            if (pk == 4 && nf >= 1 && nf <= PRED_LDS4_MAX_F) {
+            if (m->pred.nodes) {
+                run_predict(m, d_rows, n, d_margin, mode, d_out);
+                return;
+            }
+            if (nf >= 1 && nf <= PRED_LDS4_MAX_F) {
                 const uint32_t lb = (uint32_t)((n + PRED_LDS_ROWS - 1) / PRED_LDS_ROWS);
                 hipLaunchKernelGGL(predict_lds4_kernel, dim3(lb), dim3(PRED_LDS_ROWS * PRED_WAVES),
                                    (size_t)PRED_LDS_ROWS * ((nf | 1u) + PRED_RUN) * 4, m->stream,
                                    m->d_pred, m->d_nodes, m->d_cats, m->d_roots, m->n_trees,
                                    d_rows, n, nf, d_margin, m->bias, mode, d_out);
-            } else if (pk >= 1 && nf >= 1 && nf <= PRED_LDS_MAX_F) {
-                const uint32_t lb = (uint32_t)((n + PRED_LDS_ROWS - 1) / PRED_LDS_ROWS);
-                hipLaunchKernelGGL(predict_lds_kernel, dim3(lb), dim3(PRED_LDS_ROWS),
-                                   (size_t)PRED_LDS_ROWS * (nf | 1u) * 4, m->stream, m->d_pred,
-                                   m->d_nodes, m->d_cats, m->d_roots, m->n_trees, d_rows, n, nf,
-                                   d_margin, m->bias, mode, d_out);
             } else {
                 hipLaunchKernelGGL(predict_kernel, dim3(blocks), dim3(PRED_TPB), 0, m->stream,
                                    m->d_pred, m->d_nodes, m->d_cats, m->d_roots, m->n_trees, d_rows,
@@ -1215,6 +1315,7 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         double rm_sum = 0.0;
         PathBuild pb;
         pb.ok = n_features <= SHAP_PATHS_MAX_F;
+        PredBuild pt(n_features, tree_offsets, n_trees, cat_len);
         for (uint32_t t = 0; t < n_trees; t++) {
             const uint32_t b = tree_offsets[t], e = tree_offsets[t + 1];
             if (e <= b) throw ShapError(FBH_INPUT_ERROR, "tree " + std::to_string(t) + " has no nodes");
@@ -1292,6 +1393,7 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
                                                      std::to_string(MAX_SHAP_UNIQUE) +
                                                      " distinct features");
             pb.add_tree(nodes, b);
+            pt.add_tree(nodes, b, e - b, cat_words);
             rm_sum += root_mean(L, R, lv, hs, lf, b, 0);
             node_means(L, R, lv, hs, lf, b, 0, means);
         }
@@ -1306,15 +1408,28 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         m->n_nodes = total;
         m->bias = bias;
         m->root_mean = (float)rm_sum;
-        m->d_nodes = m->upload(nodes, "shap nodes");
-        m->d_rec = m->upload(rec, "shap node records");
-        m->d_pred = m->upload(pred, "walk nodes");
-        m->d_means = m->upload(means, "node means");
-        m->d_roots = m->upload(roots, "shap roots");
-        m->d_uoff = m->upload(uoff, "shap features");
-        m->d_ufeats = m->upload(ufeats, "shap features");
-        m->d_cats = m->upload(cw, "shap categories");
-        m->d_rule = m->upload(rv, "shap rule");
+        m->d_nodes = m->upload(nodes, "model arrays");
+        m->d_rec = m->upload(rec, "model arrays");
+        m->d_pred = m->upload(pred, "model arrays");
+        m->d_means = m->upload(means, "model arrays");
+        m->d_roots = m->upload(roots, "model arrays");
+        m->d_uoff = m->upload(uoff, "model arrays");
+        m->d_ufeats = m->upload(ufeats, "model arrays");
+        m->d_cats = m->upload(cw, "model arrays");
+        m->d_rule = m->upload(rv, "model arrays");
+        if (pt.ok && n_trees) {
+            pt.nodes.resize(pt.nodes.size() + 1);  // a run's last pair may be half
+            PredTrees &q = m->pred;
+            q.runs = m->upload(pt.runs, "model arrays");
+            q.ids = m->upload(pt.ids, "model arrays");
+            q.categorical = pt.categorical;
+            q.n_trees = n_trees;
+            q.n_runs = (uint32_t)pt.runs.size();
+            q.n_features = n_features;
+            q.groups = pt.groups;
+            q.most_nodes = pt.most_nodes;
+            q.nodes = m->upload(pt.nodes, "model arrays");
+        }
         if (pb.ok && !pb.nodes.empty() && m->cover_error.empty()) {
             uint32_t most = 0;
             for (uint32_t t = 0; t < n_trees; t++) most = std::max(most, pb.first[t + 1] - pb.first[t]);
@@ -1323,8 +1438,8 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
             pb.nodes.resize(pb.nodes.size() + 1);
             pb.tests.resize(pb.tests.size() + 8);
             ShapPaths &q = m->paths;
-            q.tests = m->upload(pb.tests, "path tests");
-            q.first = m->upload(pb.first, "path trees");
+            q.tests = m->upload(pb.tests, "model arrays");
+            q.first = m->upload(pb.first, "model arrays");
             q.cats = m->d_cats;
             q.n_trees = n_trees;
             q.n_features = n_features;
@@ -1333,7 +1448,7 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
             q.runs = (n_trees + q.run_trees - 1) / q.run_trees;
             q.bias = bias;
             q.root_mean = m->root_mean;
-            q.nodes = m->upload(pb.nodes, "path nodes");
+            q.nodes = m->upload(pb.nodes, "model arrays");
         }
         *out = m.release();
     });
