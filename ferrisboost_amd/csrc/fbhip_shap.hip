@@ -26,6 +26,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -770,24 +771,42 @@ struct fbh_shap_model {
     void *work = nullptr;     // both files' workspace, kept between calls
     uint64_t work_bytes = 0;
     std::mutex work_mu;       // held while the kernels that share it are enqueued
+    // Host calls: device staging of up to KEEP_STAGING bytes, and page-locked
+    // memory that the kernels of small calls read and write in place, both kept
+    // between calls; host_mu is held by the call that uses them.
+    std::mutex host_mu;
+    void *staging = nullptr, *pinned = nullptr;
+    uint64_t staging_bytes = 0;
 
     ~fbh_shap_model() {
         if (device >= 0) (void)hipSetDevice(device);
         if (stream) (void)hipStreamSynchronize(stream);
         for (void *p : allocs) (void)hipFree(p);
         if (work) (void)hipFree(work);
+        if (staging) (void)hipFree(staging);
+        if (pinned) (void)hipHostFree(pinned);
         if (e0) (void)hipEventDestroy(e0);
         if (e1) (void)hipEventDestroy(e1);
         if (stream) (void)hipStreamDestroy(stream);
     }
-    template <class T>
-    T *upload(const std::vector<T> &v, const char *what) {
+    // The arrays added so far, laid out in one allocation and sent in one copy.
+    struct Arrays {
+        std::vector<unsigned char> bytes;
+        std::vector<std::function<void(unsigned char *)>> place;
+        template <class T, class P>
+        void add(const std::vector<T> &v, P *&to) {
+            const size_t off = (bytes.size() + 255) & ~size_t(255);
+            bytes.resize(off + std::max<size_t>(sizeof(T) * v.size(), 64));
+            if (!v.empty()) std::memcpy(bytes.data() + off, v.data(), sizeof(T) * v.size());
+            place.push_back([&to, off](unsigned char *base) { to = reinterpret_cast<P *>(base + off); });
+        }
+    };
+    void upload(const Arrays &a) {
         void *p = nullptr;
-        const size_t bytes = std::max<size_t>(sizeof(T) * v.size(), 64);
-        chk(hipMalloc(&p, bytes), what);
+        chk(hipMalloc(&p, a.bytes.size()), "model arrays");
         allocs.push_back(p);
-        if (!v.empty()) chk(hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice), what);
-        return static_cast<T *>(p);
+        chk(hipMemcpy(p, a.bytes.data(), a.bytes.size(), hipMemcpyHostToDevice), "model arrays");
+        for (const auto &f : a.place) f(static_cast<unsigned char *>(p));
     }
 };
 
@@ -1234,25 +1253,76 @@ void run_host(fbh_shap_model *m, Kind k, const Staging &st, const float *rows, u
     m->last_ms = kernel_ms;
 }
 
-// Host call with staging buffers allocated for the call: batches of at most
-// 512 MiB of inputs and outputs (GpuExplainModel::compute batching,
-// src/backend/cuda/explain.rs:491-560).
+// Most staging a model keeps between host calls, and the most bytes of rows,
+// margins and outputs of a call that runs on page-locked memory. A copy of few
+// bytes costs about 15 us of launch and wait each way; a kernel fetches them
+// over the link in a few microseconds.
+constexpr uint64_t KEEP_STAGING = 128ull << 20;
+constexpr uint64_t PINNED_BYTES = 256ull << 10;
+
+uint64_t round256(uint64_t v) { return (v + 255) & ~uint64_t(255); }
+
+// Whether the kind's kernels read a row a few times in order and write each
+// output once.
+bool runs_in_place(const fbh_shap_model *m, Kind k) {
+    if (k == Kind::Contribs) return takes_paths(m, false);
+    return (k == Kind::Margin || k == Kind::Value || k == Kind::Leaf) && m->pred.nodes;
+}
+
+// Host call: batches of at most 512 MiB of inputs and outputs
+// (GpuExplainModel::compute batching, src/backend/cuda/explain.rs:491-560)
+// through the model's staging, or through staging of its own where another
+// thread's call has that or the call needs more than is kept.
 void run_host_alloc(fbh_shap_model *m, Kind k, const float *rows, uint64_t n_rows,
                     const float *margin, float *out) {
     if (!m || (!rows && n_rows) || (!out && n_rows)) throw ShapError(FBH_INPUT_ERROR, "null argument");
     check_kind(m, k);
     if (n_rows == 0) return;
     chk(hipSetDevice(m->device), "hipSetDevice");
-    const uint64_t w = out_width(m, k);
-    const uint64_t per_row = 4ull * (m->n_features + 1 + w);
+    const uint64_t w = out_width(m, k), nf = m->n_features;
+    const uint64_t per_row = 4ull * (nf + 1 + w);
+    std::unique_lock<std::mutex> mine(m->host_mu, std::try_to_lock);
+    if (mine && n_rows <= PINNED_BYTES / per_row && runs_in_place(m, k)) {
+        if (!m->pinned) chk(hipHostMalloc(&m->pinned, PINNED_BYTES + 1024, hipHostMallocDefault), "pinned");
+        float *x = static_cast<float *>(m->pinned);
+        float *mg = x + round256(4 * n_rows * nf) / 4, *o = mg + round256(4 * n_rows) / 4;
+        std::memcpy(x, rows, 4 * n_rows * nf);
+        if (margin) std::memcpy(mg, margin, 4 * n_rows);
+        chk(hipEventRecord(m->e0, m->stream), "event");
+        enqueue(m, k, x, n_rows, margin ? mg : nullptr, o);
+        chk(hipEventRecord(m->e1, m->stream), "event");
+        chk(hipStreamSynchronize(m->stream), "explain");
+        std::memcpy(out, o, 4 * n_rows * w);
+        float ms = 0.0f;
+        chk(hipEventElapsedTime(&ms, m->e0, m->e1), "event");
+        m->last_ms = ms;
+        return;
+    }
     Staging st;
     st.cap_rows = std::min<uint64_t>(n_rows, std::max<uint64_t>(1, (512ull << 20) / per_row));
-    chk(hipMalloc(&st.rows, 4 * st.cap_rows * m->n_features + 4), "staging rows");
-    std::unique_ptr<float, decltype(&hipFree)> f1(st.rows, hipFree);
-    chk(hipMalloc(&st.out, 4 * st.cap_rows * w + 4), "staging output");
-    std::unique_ptr<float, decltype(&hipFree)> f2(st.out, hipFree);
-    if (margin) chk(hipMalloc(&st.margin, 4 * st.cap_rows), "staging margin");
-    std::unique_ptr<float, decltype(&hipFree)> f3(st.margin, hipFree);
+    const uint64_t o_rows = round256(4 * st.cap_rows * nf);
+    const uint64_t o_out = o_rows + round256(4 * st.cap_rows);
+    const uint64_t need = o_out + 4 * st.cap_rows * w + 4;
+    std::unique_ptr<void, decltype(&hipFree)> own(nullptr, hipFree);
+    unsigned char *base;
+    if (mine && need <= KEEP_STAGING) {
+        if (m->staging_bytes < need) {
+            if (m->staging) chk(hipFree(m->staging), "staging");
+            m->staging = nullptr;
+            m->staging_bytes = 0;
+            chk(hipMalloc(&m->staging, need), "staging");
+            m->staging_bytes = need;
+        }
+        base = static_cast<unsigned char *>(m->staging);
+    } else {
+        void *p = nullptr;
+        chk(hipMalloc(&p, need), "staging");
+        own.reset(p);
+        base = static_cast<unsigned char *>(p);
+    }
+    st.rows = reinterpret_cast<float *>(base);
+    st.margin = reinterpret_cast<float *>(base + o_rows);
+    st.out = reinterpret_cast<float *>(base + o_out);
     run_host(m, k, st, rows, n_rows, margin, out);
 }
 
@@ -1274,8 +1344,6 @@ void *scratch_of(int device) {
     }
     return g_scratch_ptr[device];
 }
-
-uint64_t round256(uint64_t v) { return (v + 255) & ~uint64_t(255); }
 
 }  // namespace
 
@@ -1408,27 +1476,28 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         m->n_nodes = total;
         m->bias = bias;
         m->root_mean = (float)rm_sum;
-        m->d_nodes = m->upload(nodes, "model arrays");
-        m->d_rec = m->upload(rec, "model arrays");
-        m->d_pred = m->upload(pred, "model arrays");
-        m->d_means = m->upload(means, "model arrays");
-        m->d_roots = m->upload(roots, "model arrays");
-        m->d_uoff = m->upload(uoff, "model arrays");
-        m->d_ufeats = m->upload(ufeats, "model arrays");
-        m->d_cats = m->upload(cw, "model arrays");
-        m->d_rule = m->upload(rv, "model arrays");
+        fbh_shap_model::Arrays arrays;
+        arrays.add(nodes, m->d_nodes);
+        arrays.add(rec, m->d_rec);
+        arrays.add(pred, m->d_pred);
+        arrays.add(means, m->d_means);
+        arrays.add(roots, m->d_roots);
+        arrays.add(uoff, m->d_uoff);
+        arrays.add(ufeats, m->d_ufeats);
+        arrays.add(cw, m->d_cats);
+        arrays.add(rv, m->d_rule);
         if (pt.ok && n_trees) {
             pt.nodes.resize(pt.nodes.size() + 1);  // a run's last pair may be half
             PredTrees &q = m->pred;
-            q.runs = m->upload(pt.runs, "model arrays");
-            q.ids = m->upload(pt.ids, "model arrays");
+            arrays.add(pt.runs, q.runs);
+            arrays.add(pt.ids, q.ids);
             q.categorical = pt.categorical;
             q.n_trees = n_trees;
             q.n_runs = (uint32_t)pt.runs.size();
             q.n_features = n_features;
             q.groups = pt.groups;
             q.most_nodes = pt.most_nodes;
-            q.nodes = m->upload(pt.nodes, "model arrays");
+            arrays.add(pt.nodes, q.nodes);
         }
         if (pb.ok && !pb.nodes.empty() && m->cover_error.empty()) {
             uint32_t most = 0;
@@ -1438,9 +1507,9 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
             pb.nodes.resize(pb.nodes.size() + 1);
             pb.tests.resize(pb.tests.size() + 8);
             ShapPaths &q = m->paths;
-            q.tests = m->upload(pb.tests, "model arrays");
-            q.first = m->upload(pb.first, "model arrays");
-            q.cats = m->d_cats;
+            arrays.add(pb.tests, q.tests);
+            arrays.add(pb.first, q.first);
+            arrays.add(cw, q.cats);
             q.n_trees = n_trees;
             q.n_features = n_features;
             q.stride = (most + 8) & ~7u;
@@ -1448,8 +1517,9 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
             q.runs = (n_trees + q.run_trees - 1) / q.run_trees;
             q.bias = bias;
             q.root_mean = m->root_mean;
-            q.nodes = m->upload(pb.nodes, "model arrays");
+            arrays.add(pb.nodes, q.nodes);
         }
+        m->upload(arrays);
         *out = m.release();
     });
 }

@@ -3,9 +3,13 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <future>
 #include <limits>
 #include <memory>
+#include <mutex>
 #include <string>
+#include <thread>
+#include <utility>
 
 #include "fbhip.h"
 #include "fbt_internal.h"
@@ -19,8 +23,56 @@ uint32_t last_round_stats(double *wall, double *ms, uint64_t *bytes, uint32_t ca
 uint32_t last_round_launches(uint64_t *launches, uint32_t cap);
 }  // namespace fbt
 
+namespace {
+
+using ShapModel = std::unique_ptr<fbh_shap_model, int (*)(fbh_shap_model *)>;
+
+// The device models of a model's trees that predictions and explanations have
+// used, kept for the next call: one for a tree range, output and device. A call
+// takes its entry out and puts it back, so that calls from several threads each
+// work on a device model of their own; the oldest beyond KEEP are dropped.
+class DeviceModels {
+public:
+    struct Key {
+        uint32_t begin, end, output;  // output of a multi-output model, or ALL
+        int device;
+        bool operator==(const Key &o) const {
+            return begin == o.begin && end == o.end && output == o.output && device == o.device;
+        }
+    };
+    static constexpr uint32_t ALL = 0xFFFFFFFFu;
+
+    ShapModel take(const Key &k) {
+        std::lock_guard<std::mutex> g(mu_);
+        for (size_t i = 0; i < kept_.size(); i++)
+            if (kept_[i].first == k) {
+                ShapModel m = std::move(kept_[i].second);
+                kept_.erase(kept_.begin() + (ptrdiff_t)i);
+                return m;
+            }
+        return ShapModel(nullptr, fbh_shap_model_destroy);
+    }
+    void put(const Key &k, ShapModel m) {
+        ShapModel old(nullptr, fbh_shap_model_destroy);  // destroyed outside the lock
+        std::lock_guard<std::mutex> g(mu_);
+        kept_.emplace_back(k, std::move(m));
+        if (kept_.size() > KEEP) {
+            old = std::move(kept_.front().second);
+            kept_.erase(kept_.begin());
+        }
+    }
+
+private:
+    static constexpr size_t KEEP = 8;
+    std::mutex mu_;
+    std::vector<std::pair<Key, ShapModel>> kept_;
+};
+
+}  // namespace
+
 struct fbt_model {
     fbt::Model m;
+    mutable DeviceModels device;
 };
 
 namespace {
@@ -244,8 +296,6 @@ namespace {
 // The device explanation model of trees [begin, end) (GpuExplainModel::new,
 // src/backend/cuda/explain.rs:186-490, over the model slice that
 // iteration_range selects, src/python/mod.rs:1993-2029).
-using ShapModel = std::unique_ptr<fbh_shap_model, int (*)(fbh_shap_model *)>;
-
 void backend_fail(int rc) {
     char buf[1024];
     fbh_last_error(buf, sizeof(buf));
@@ -287,11 +337,83 @@ ShapModel explain_model(const fbt::Model &m, const std::vector<uint32_t> &ids, f
     return ShapModel(sm, fbh_shap_model_destroy);
 }
 
-ShapModel explain_model(const fbt::Model &m, uint32_t begin, uint32_t end, int device) {
-    std::vector<uint32_t> ids;
-    for (uint32_t t = begin; t < end; t++) ids.push_back(t);
-    return explain_model(m, ids, m.base_margin(), device);
+// A call's use of the device model of the trees [begin, end) (of output `output`
+// alone, or of all): the kept one, or a new one, kept afterwards.
+class DeviceModel {
+public:
+    DeviceModel(const fbt_model &mm, uint32_t begin, uint32_t end, uint32_t output, int device)
+        : owner_(mm.device), key_{begin, end, output, device}, m_(mm.device.take(key_)) {
+        if (m_) return;
+        const bool all = output == DeviceModels::ALL;
+        const uint32_t K = mm.m.n_outputs();
+        std::vector<uint32_t> ids;
+        for (uint32_t t = begin; t < end; t++)
+            if (all || t % K == output) ids.push_back(t);
+        m_ = explain_model(mm.m, ids, all ? mm.m.base_margin() : mm.m.class_margins[output], device);
+    }
+    ~DeviceModel() {
+        try {
+            owner_.put(key_, std::move(m_));
+        } catch (...) {  // out of memory: the device model goes
+        }
+    }
+    DeviceModel(const DeviceModel &) = delete;
+    DeviceModel &operator=(const DeviceModel &) = delete;
+    fbh_shap_model *get() const { return m_.get(); }
+
+private:
+    DeviceModels &owner_;
+    DeviceModels::Key key_;
+    ShapModel m_;
+};
+
+// Whether any of the cells is the largest float32. Blocks without an early exit,
+// which the compiler vectorises.
+__attribute__((optimize("O3"))) bool holds_reserved(const float *x, uint64_t n) {
+    constexpr uint64_t BLOCK = 4096;
+    for (uint64_t b = 0; b < n; b += BLOCK) {
+        const uint64_t e = std::min(n, b + BLOCK);
+        uint32_t found = 0;
+        for (uint64_t i = b; i < e; i++)
+            found |= x[i] == std::numeric_limits<float>::max() ? 1u : 0u;
+        if (found) return true;
+    }
+    return false;
 }
+
+// Feature values equal to f32::MAX are reserved for split boundaries
+// (src/model/tree.rs:985-990) and rejected, as in training. Large inputs are
+// looked through by threads while the device works; the call's result counts
+// only once check() has returned.
+class ReservedCheck {
+public:
+    ReservedCheck(const float *x, uint64_t n) {
+        constexpr uint64_t SHARE = 1u << 18;  // cells worth a thread
+        const uint64_t hw = std::max(1u, std::thread::hardware_concurrency());
+        const uint64_t k = std::min<uint64_t>({n / SHARE, hw, 8});
+        if (k == 0) {
+            found_ = holds_reserved(x, n);
+            if (found_) check();
+            return;
+        }
+        for (uint64_t i = 0; i < k; i++) {
+            const uint64_t b = n * i / k, e = n * (i + 1) / k;
+            parts_.push_back(std::async(std::launch::async, [=] { return holds_reserved(x + b, e - b); }));
+        }
+    }
+    void check() {
+        for (auto &p : parts_) found_ |= p.get();
+        parts_.clear();
+        if (found_)
+            throw fbt::InputError(
+                "feature values equal to the largest float32 (3.4028235e38) are reserved "
+                "and cannot be scored");
+    }
+
+private:
+    std::vector<std::future<bool>> parts_;
+    bool found_ = false;
+};
 
 // softmax_in_place (src/training/objective.rs:1308-1322): the row's largest
 // margin, the double sum of expf(v - max) in order, each value divided by
@@ -338,13 +460,14 @@ constexpr uint64_t HOST_ORDER_ROWS = 512;
 // A multiclass model's outputs: each class scored or explained by its own
 // trees with its own intercept (Model::class_view, src/model/tree.rs:
 // 395-425), the per-class results laid out [row][class][...].
-void predict_multiclass(const fbt::Model &m, const float *x, uint64_t n_rows, uint32_t nf,
+void predict_multiclass(const fbt_model &mm, const float *x, uint64_t n_rows, uint32_t nf,
                         uint32_t output, uint32_t begin, uint32_t end, const float *base_margin,
                         int device, float *out) {
+    const fbt::Model &m = mm.m;
     const uint32_t K = m.n_outputs();
     if (output == FBT_OUT_LEAF) {
         if (device < 0) throw fbt::InputError("explanations run on the device; pass a device index");
-        ShapModel sm = explain_model(m, begin, end, device);
+        DeviceModel sm(mm, begin, end, DeviceModels::ALL, device);
         if (int rc = fbh_predict(sm.get(), x, n_rows, nullptr, FBH_PREDICT_LEAF, out)) backend_fail(rc);
         g_last_shap_ms = fbh_shap_last_ms(sm.get());
         return;
@@ -358,21 +481,17 @@ void predict_multiclass(const fbt::Model &m, const float *x, uint64_t n_rows, ui
     std::vector<float> margins(scores ? n_rows * K : 0), col(n_rows * width);
     double ms = 0.0;
     for (uint32_t k = 0; k < K; k++) {
-        std::vector<uint32_t> ids;
-        for (uint32_t t = begin; t < end; t++)
-            if (t % K == k) ids.push_back(t);
         const float *bm = base_margin ? base_margin + (uint64_t)k * n_rows : nullptr;
-        const float bias = m.class_margins[k];
         if (device < 0) {
             for (uint64_t r = 0; r < n_rows; r++) {
-                float acc = bm ? bm[r] : bias;
-                for (uint32_t t : ids) acc += m.trees[t].leaf_value(x + r * nf);
+                float acc = bm ? bm[r] : m.class_margins[k];
+                for (uint32_t t = begin; t < end; t++)
+                    if (t % K == k) acc += m.trees[t].leaf_value(x + r * nf);
                 col[r] = acc;
             }
         } else {
-            ShapModel sm = explain_model(m, ids, bias, device);
-            int rc = FBH_OK;
-            if (!scores && n_rows < HOST_ORDER_ROWS) rc = fbh_shap_set_host_order(sm.get(), 1);
+            DeviceModel sm(mm, begin, end, k, device);
+            int rc = fbh_shap_set_host_order(sm.get(), !scores && n_rows < HOST_ORDER_ROWS);
             if (rc) backend_fail(rc);
             if (scores) rc = fbh_predict(sm.get(), x, n_rows, bm, FBH_PREDICT_MARGIN, col.data());
             else if (output == FBT_OUT_CONTRIBS) rc = fbh_shap_contribs(sm.get(), x, n_rows, bm, col.data());
@@ -404,6 +523,52 @@ void predict_multiclass(const fbt::Model &m, const float *x, uint64_t n_rows, ui
     }
 }
 
+// A single-output model's outputs.
+void predict_single(const fbt_model &mm, const float *x, uint64_t n_rows, uint32_t nf,
+                    uint32_t output, uint32_t begin, uint32_t end, const float *base_margin,
+                    int device, float *out) {
+    const fbt::Model &m = mm.m;
+    const bool logistic = m.objective == 1;
+    if (device < 0) {
+        // Host scoring (use_gpu=False): Model::predict_margin_upto and the
+        // objective's transform with the host libm.
+        if (output != FBT_OUT_MARGIN && output != FBT_OUT_VALUE)
+            throw fbt::InputError("explanations run on the device; pass a device index");
+        const float bm = m.base_margin();
+        for (uint64_t r = 0; r < n_rows; r++) {
+            float acc = base_margin ? base_margin[r] : bm;
+            for (uint32_t t = begin; t < end; t++) acc += m.trees[t].leaf_value(x + r * nf);
+            out[r] = output == FBT_OUT_VALUE && logistic ? 1.0f / (1.0f + std::exp(-acc)) : acc;
+        }
+        return;
+    }
+    DeviceModel sm(mm, begin, end, DeviceModels::ALL, device);
+    int rc = FBH_OK;
+    switch (output) {
+        case FBT_OUT_MARGIN:
+            rc = fbh_predict(sm.get(), x, n_rows, base_margin, FBH_PREDICT_MARGIN, out);
+            break;
+        case FBT_OUT_VALUE:
+            rc = fbh_predict(sm.get(), x, n_rows, base_margin,
+                             logistic ? FBH_PREDICT_SIGMOID : FBH_PREDICT_MARGIN, out);
+            break;
+        case FBT_OUT_LEAF:
+            rc = fbh_predict(sm.get(), x, n_rows, nullptr, FBH_PREDICT_LEAF, out);
+            break;
+        case FBT_OUT_CONTRIBS:
+            rc = fbh_shap_contribs(sm.get(), x, n_rows, base_margin, out);
+            break;
+        case FBT_OUT_APPROX_CONTRIBS:
+            rc = fbh_saabas_contribs(sm.get(), x, n_rows, base_margin, out);
+            break;
+        default:
+            rc = fbh_shap_interactions(sm.get(), x, n_rows, base_margin, out);
+            break;
+    }
+    if (rc) backend_fail(rc);
+    g_last_shap_ms = fbh_shap_last_ms(sm.get());
+}
+
 }  // namespace
 
 extern "C" {
@@ -428,61 +593,21 @@ int fbt_predict(const fbt_model *mm, const float *x, uint64_t n_rows, uint32_t n
             throw fbt::InputError("tree range [" + std::to_string(tree_begin) + ", " +
                                   std::to_string(tree_end) + ") is outside the model's " +
                                   std::to_string(m.trees.size()) + " trees");
-        // Feature values equal to f32::MAX are reserved for split boundaries
-        // (src/model/tree.rs:985-990) and rejected, as in training.
-        const uint64_t cells = n_rows * (uint64_t)n_features;
-        for (uint64_t i = 0; i < cells; i++)
-            if (x[i] == std::numeric_limits<float>::max())
-                throw fbt::InputError(
-                    "feature values equal to the largest float32 (3.4028235e38) are reserved "
-                    "and cannot be scored");
-        if (m.n_outputs() > 1) {
-            predict_multiclass(m, x, n_rows, n_features, output, tree_begin, tree_end, base_margin,
-                               device, out);
-            return;
+        ReservedCheck reserved(x, n_rows * (uint64_t)n_features);
+        try {
+            if (m.n_outputs() > 1)
+                predict_multiclass(*mm, x, n_rows, n_features, output, tree_begin, tree_end,
+                                   base_margin, device, out);
+            else
+                predict_single(*mm, x, n_rows, n_features, output, tree_begin, tree_end,
+                               base_margin, device, out);
+        } catch (...) {
+            reserved.check();  // a reserved value is the error to report
+            throw;
         }
-        const bool logistic = m.objective == 1;
-        if (device < 0) {
-            // Host scoring (use_gpu=False): Model::predict_margin_upto and the
-            // objective's transform with the host libm.
-            if (output != FBT_OUT_MARGIN && output != FBT_OUT_VALUE)
-                throw fbt::InputError("explanations run on the device; pass a device index");
-            const float bm = m.base_margin();
-            for (uint64_t r = 0; r < n_rows; r++) {
-                float acc = base_margin ? base_margin[r] : bm;
-                for (uint32_t t = tree_begin; t < tree_end; t++) acc += m.trees[t].leaf_value(x + r * n_features);
-                out[r] = output == FBT_OUT_VALUE && logistic ? 1.0f / (1.0f + std::exp(-acc)) : acc;
-            }
-            return;
-        }
-        ShapModel sm = explain_model(m, tree_begin, tree_end, device);
-        int rc = FBH_OK;
-        switch (output) {
-            case FBT_OUT_MARGIN:
-                rc = fbh_predict(sm.get(), x, n_rows, base_margin, FBH_PREDICT_MARGIN, out);
-                break;
-            case FBT_OUT_VALUE:
-                rc = fbh_predict(sm.get(), x, n_rows, base_margin,
-                                 logistic ? FBH_PREDICT_SIGMOID : FBH_PREDICT_MARGIN, out);
-                break;
-            case FBT_OUT_LEAF:
-                rc = fbh_predict(sm.get(), x, n_rows, nullptr, FBH_PREDICT_LEAF, out);
-                break;
-            case FBT_OUT_CONTRIBS:
-                rc = fbh_shap_contribs(sm.get(), x, n_rows, base_margin, out);
-                break;
-            case FBT_OUT_APPROX_CONTRIBS:
-                rc = fbh_saabas_contribs(sm.get(), x, n_rows, base_margin, out);
-                break;
-            default:
-                rc = fbh_shap_interactions(sm.get(), x, n_rows, base_margin, out);
-                break;
-        }
-        if (rc) backend_fail(rc);
-        g_last_shap_ms = fbh_shap_last_ms(sm.get());
+        reserved.check();
     });
 }
-
 int fbt_model_from_json(const char *json, size_t len, fbt_model **out) {
     return guard([&] {
         if (!json || !out) throw fbt::InputError("null argument");
