@@ -215,6 +215,8 @@ struct fbh_ctx {
     float *d_cut_values = nullptr;
     float *rows_stage = nullptr;
     bool cuts_set = false;
+    uint8_t *pack_tab = nullptr;  // pack_rows's tables
+    uint64_t pack_tab_bytes = 0;
     // Device binning under a plan that does not keep the bin columns: a
     // chunk's bins land in bin_stage (feature f's column of stage_rows()
     // cells at byte bin_off[f], 256-aligned), resident tiles are packed from
@@ -1361,6 +1363,43 @@ int fbh_upload_block(fbh_ctx *c, const uint32_t *feat_ids, uint32_t n_feats, uin
     });
 }
 
+// Rows of the given layouts from the resident bin columns in one launch, through
+// a device table kept for the next time; false (nothing done) when the budget has
+// no room for the table.
+struct RowLayout {
+    uint8_t *out;
+    uint32_t pitch;
+    std::vector<std::pair<uint32_t, uint32_t>> cells;  // feature, offset in the row
+};
+
+static bool pack_rows(fbh_ctx &c, const std::vector<RowLayout> &layouts) {
+    if (layouts.empty()) return true;
+    std::vector<PackRowsDev> rows;
+    std::vector<PackCellDev> cells;
+    for (const RowLayout &l : layouts) {
+        rows.push_back({l.out, l.pitch, (uint32_t)cells.size(), (uint32_t)l.cells.size()});
+        for (const auto &f : l.cells) cells.push_back({c.cols[f.first], c.width[f.first], f.second});
+    }
+    const uint64_t at = al256(sizeof(PackRowsDev) * rows.size());
+    const uint64_t bytes = at + sizeof(PackCellDev) * cells.size();
+    if (c.pack_tab_bytes < bytes) {
+        if (c.device_bytes + bytes + 256 > c.plan.budget) return false;
+        c.release_alloc(c.pack_tab);
+        c.pack_tab = c.alloc<uint8_t>(bytes, "row packing table");
+        c.pack_tab_bytes = bytes;
+    }
+    std::vector<uint8_t> tab(bytes);
+    std::memcpy(tab.data(), rows.data(), sizeof(PackRowsDev) * rows.size());
+    std::memcpy(tab.data() + at, cells.data(), sizeof(PackCellDev) * cells.size());
+    check(hipMemcpyAsync(c.pack_tab, tab.data(), bytes, hipMemcpyHostToDevice, c.stream),
+          "row packing table");
+    check(launch_pack_rows(reinterpret_cast<const PackRowsDev *>(c.pack_tab), (uint32_t)rows.size(),
+                           reinterpret_cast<const PackCellDev *>(c.pack_tab + at), c.n_rows, c.stream),
+          "row packing");
+    c.sync();  // the host table goes, and the device table may be rewritten
+    return true;
+}
+
 int fbh_set_cuts(fbh_ctx *c, const float *cut_values, const uint32_t *cut_offsets,
                  const uint8_t *categorical) {
     return guard([&] {
@@ -1507,22 +1546,33 @@ int fbh_finish_rows(fbh_ctx *c) {
         check(hipSetDevice(c->device), "hipSetDevice");
         c->tm_stale = true;
         c->hot_ready = false;
-        for (uint32_t f = 0; f < c->n_features; f++) {
-            const fbh_ctx::Tile &t = c->tiles[c->feat_tile[f]];
-            if (!c->plan.columns_resident) {
-                // packed chunk by chunk as the rows came (pack_staged_rows)
-            } else if (t.resident) {
-                const uint32_t off = (uint32_t)c->feat_pos[f] * c->width[f];
-                check(launch_pack_feature(c->cols[f], c->n_rows, c->width[f], t.data, t.stride,
-                                          off, c->stream),
-                      "tile packing");
-            } else {
-                // A streamed tile's records live in pinned host memory: bring
-                // the column back and lay it into them as fbh_upload_block does.
-                throw InputError("device binning needs every tile resident");
+        // Without resident columns the records were packed chunk by chunk as the
+        // rows came (pack_staged_rows).
+        if (c->plan.columns_resident) {
+            std::vector<RowLayout> layouts(c->bundles.size());
+            for (size_t b = 0; b < c->bundles.size(); b++)
+                layouts[b] = {c->bundles[b].data, c->bundles[b].pitch, {}};
+            for (const auto &t : c->tiles) {
+                // A streamed tile's records live in pinned host memory: the
+                // columns would have to come back as fbh_upload_block's do.
+                if (!t.resident) throw InputError("device binning needs every tile resident");
+                if (t.bundle < 0) layouts.push_back({t.data, t.stride, {}});
+                RowLayout &l = t.bundle < 0 ? layouts.back() : layouts[(size_t)t.bundle];
+                for (uint32_t f : t.feats)
+                    l.cells.emplace_back(f, (t.bundle < 0 ? 0 : t.bundle_off) +
+                                                (uint32_t)c->feat_pos[f] * t.width);
             }
-            c->uploaded[f] = 1;
+            bool fits = true;
+            for (const RowLayout &l : layouts) fits &= l.pitch <= 128 && l.pitch % 4 == 0;
+            if (!fits || !pack_rows(*c, layouts))
+                for (uint32_t f = 0; f < c->n_features; f++) {
+                    const fbh_ctx::Tile &t = c->tiles[c->feat_tile[f]];
+                    check(launch_pack_feature(c->cols[f], c->n_rows, c->width[f], t.data, t.stride,
+                                              (uint32_t)c->feat_pos[f] * c->width[f], c->stream),
+                          "tile packing");
+                }
         }
+        for (uint32_t f = 0; f < c->n_features; f++) c->uploaded[f] = 1;
         c->pack_sig.clear();
         c->sync();
     });
@@ -1547,15 +1597,21 @@ bool ensure_tile_major(fbh_ctx &c, const std::vector<const fbh_ctx::Tile *> &til
     for (const fbh_ctx::Tile *t : tiles)
         if (!t->tm) need += std::max<uint64_t>((uint64_t)t->rec * c.n_rows, 256);
     if (need && c.device_bytes + need + 256 > c.plan.budget) return false;
+    std::vector<RowLayout> layouts;
     for (const fbh_ctx::Tile *tp : tiles) {
         fbh_ctx::Tile &t = c.tiles[tp - c.tiles.data()];
         if (t.tm) continue;
         t.tm = c.alloc<uint8_t>((uint64_t)t.rec * c.n_rows, "tile-major records");
+        layouts.push_back({t.tm, t.rec, {}});
         for (uint32_t f : t.feats)
-            check(launch_pack_feature(c.cols[f], c.n_rows, t.width, t.tm, t.rec,
-                                      (uint32_t)c.feat_pos[f] * t.width, c.stream),
-                  "tile-major packing");
+            layouts.back().cells.emplace_back(f, (uint32_t)c.feat_pos[f] * t.width);
     }
+    if (!pack_rows(c, layouts))
+        for (const RowLayout &l : layouts)
+            for (const auto &f : l.cells)
+                check(launch_pack_feature(c.cols[f.first], c.n_rows, c.width[f.first], l.out, l.pitch,
+                                          f.second, c.stream),
+                      "tile-major packing");
     return true;
 }
 

@@ -567,6 +567,22 @@ struct PackTileDev {
 hipError_t launch_pack_tiles(const PackTileDev *tiles, uint32_t n_tiles, uint32_t width,
                              uint64_t n_rows, hipStream_t s);
 
+// A row layout of up to 128 bytes (a row bundle, or one tile's records) and a
+// column's cells in it.
+struct PackRowsDev {
+    uint8_t *out;           // row 0
+    uint32_t pitch;         // bytes a row (multiple of 4)
+    uint32_t first, count;  // its cells
+};
+struct PackCellDev {
+    const uint8_t *col;
+    uint32_t width;         // 1 or 2
+    uint32_t off;           // of the cell in the row
+};
+// Every layout's rows from its columns (bytes of no cell become zero).
+hipError_t launch_pack_rows(const PackRowsDev *layouts, uint32_t n_layouts, const PackCellDev *cells,
+                            uint64_t n_rows, hipStream_t s);
+
 // Categories the device split scan sorts in LDS (weights + order, 32 KiB).
 constexpr uint32_t MAX_DEVICE_CATS = 4096;
 // Distinct split features of one tree the TreeSHAP kernel accepts.
