@@ -223,7 +223,7 @@ HIP_SYMBOLS = [
     "fbh_apply_leaf_values",
     "fbh_upload_rows", "fbh_finish_rows", "fbh_sketch_device_bytes", "fbh_sketch_fits",
     "fbh_sketch_create", "fbh_sketch_push_rows", "fbh_sketch_cuts", "fbh_sketch_missing",
-    "fbh_sketch_destroy",
+    "fbh_sketch_rows", "fbh_sketch_destroy", "fbh_bin_rows",
     "fbh_upload_quantize_gpair",
     "fbh_upload_gpair_fixed", "fbh_set_objective", "fbh_set_multiclass",
     "fbh_multiclass_begin_round", "fbh_set_output", "fbh_set_quantile",
@@ -346,6 +346,9 @@ def hip() -> C.CDLL:
                                             P, C.c_uint32, C.c_uint32, C.c_float, C.POINTER(P)]
         L.fbh_shap_model_destroy.argtypes = [P]
         L.fbh_shap_set_host_order.argtypes = [P, C.c_int]
+        L.fbh_sketch_rows.argtypes = [P]
+        L.fbh_sketch_rows.restype = P
+        L.fbh_bin_rows.argtypes = [P, P, C.c_uint64, C.c_uint64]
         L.fbh_shap_contribs.argtypes = [P, P, C.c_uint64, P, P]
         L.fbh_shap_contribs_device.argtypes = [P, P, C.c_uint64, P, P, C.c_int]
         L.fbh_shap_last_ms.argtypes = [P]

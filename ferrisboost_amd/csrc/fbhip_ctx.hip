@@ -1539,6 +1539,27 @@ int fbh_upload_rows(fbh_ctx *c, const float *x, uint64_t row0, uint64_t n_rows) 
     });
 }
 
+int fbh_bin_rows(fbh_ctx *c, const float *x, uint64_t row0, uint64_t n_rows) {
+    return guard([&] {
+        if (!c || (!x && n_rows)) throw InputError("null argument");
+        if (!c->cuts_set) throw InputError("fbh_set_cuts must come before fbh_bin_rows");
+        if (row0 > c->n_rows || n_rows > c->n_rows - row0)
+            throw InputError("rows out of range");
+        if (n_rows == 0) return;
+        check(hipSetDevice(c->device), "hipSetDevice");
+        const bool staged = !c->plan.columns_resident;
+        const uint64_t cap = staged ? c->stage_rows() : n_rows, nf = c->n_features;
+        for (uint64_t r = 0; r < n_rows; r += cap) {
+            const uint64_t b = std::min(cap, n_rows - r);
+            check(launch_bin_rows(x + r * nf, b, (uint32_t)nf, staged ? 0 : row0 + r, c->d_binfeats,
+                                  c->stream),
+                  "row binning");
+            if (staged) pack_staged_rows(c, row0 + r, b);
+        }
+        c->sync();
+    });
+}
+
 int fbh_finish_rows(fbh_ctx *c) {
     return guard([&] {
         if (!c) throw InputError("null argument");

@@ -41,12 +41,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstring>
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/fbhip.h"
@@ -90,6 +92,7 @@ constexpr uint32_t SK_ROWS = 64;   // rows of a staging tile (one wave of lanes)
 constexpr uint32_t SK_FEATS = 64;  // features of a staging tile
 constexpr uint32_t SK_MAX_BIN = 1024;                   // largest max_bin sketched here
 constexpr uint64_t SK_STAGE_BYTES = 256ull << 20;      // row staging of one chunk
+constexpr uint64_t KEEP_CHUNK_BYTES = 64ull << 20;     // rows uploaded, then sketched, at a time
 
 __host__ __device__ inline uint32_t sk_limit(uint32_t max_bin) {
     const uint32_t l = 16u * max_bin;
@@ -706,6 +709,70 @@ hipError_t allow_lds(K kernel) {
                                (int)(160 * 1024 - fa.sharedSizeBytes));
 }
 
+// Large host-to-device copies through page-locked memory that two threads fill in
+// turn: 42 GB/s where a copy from pageable memory reaches 28 (one thread fills
+// 26 GB/s, more than two add nothing). A thread's two pieces of 4 MiB cost 3 ms
+// when first touched, so only matrices of PIPE_LEAST bytes take this way.
+struct RowPipe {
+    static constexpr int THREADS = 2, SLOTS = 2;
+    static constexpr uint64_t PIECE = 4ull << 20;
+    static constexpr uint64_t PIPE_LEAST = 256ull << 20;
+    unsigned char *pinned = nullptr;
+    hipEvent_t done[THREADS][SLOTS] = {};
+
+    // Enqueues the copy on `s`; src may be reused when it returns.
+    void copy(int device, void *dst, const void *src, uint64_t bytes, hipStream_t s) {
+        if (!pinned) {
+            void *p = nullptr;
+            sk_check(hipHostMalloc(&p, THREADS * SLOTS * PIECE, hipHostMallocDefault), "row pipe");
+            pinned = static_cast<unsigned char *>(p);
+            for (auto &t : done)
+                for (hipEvent_t &e : t)
+                    sk_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
+        }
+        std::atomic<uint64_t> next{0};
+        hipError_t failed[THREADS] = {};
+        auto work = [&](int t) {
+            hipError_t e = hipSetDevice(device);
+            for (int slot = 0; e == hipSuccess; slot = (slot + 1) % SLOTS) {
+                const uint64_t at = next.fetch_add(PIECE);
+                if (at >= bytes) break;
+                const uint64_t n = std::min(PIECE, bytes - at);
+                unsigned char *b = pinned + (uint64_t)(t * SLOTS + slot) * PIECE;
+                // (an event that was never recorded is complete)
+                if ((e = hipEventSynchronize(done[t][slot])) != hipSuccess) break;
+                std::memcpy(b, static_cast<const unsigned char *>(src) + at, n);
+                e = hipMemcpyAsync(static_cast<unsigned char *>(dst) + at, b, n,
+                                   hipMemcpyHostToDevice, s);
+                if (e == hipSuccess) e = hipEventRecord(done[t][slot], s);
+            }
+            failed[t] = e;
+        };
+        std::thread other(work, 1);
+        work(0);
+        other.join();
+        for (hipError_t e : failed) sk_check(e, "row upload");
+    }
+    // Once nothing of it is in flight.
+    void release() {
+        for (auto &t : done)
+            for (hipEvent_t &e : t) {
+                if (e) (void)hipEventDestroy(e);
+                e = nullptr;
+            }
+        if (pinned) (void)hipHostFree(pinned);
+        pinned = nullptr;
+    }
+};
+
+// Whether a sketch keeps its rows on the device: without a memory budget, when four
+// times the matrix (the rows beside a context's records, columns and arrays of them)
+// and the sketch fit what is free.
+bool keeps_rows(uint64_t n_rows, uint32_t nf, uint64_t need, uint64_t room, uint64_t budget) {
+    const uint64_t bytes = 4 * n_rows * nf;
+    return budget == 0 && need + 4 * bytes + 512 * n_rows <= room;
+}
+
 }  // namespace
 
 struct fbh_sketch {
@@ -716,10 +783,17 @@ struct fbh_sketch {
     std::vector<uint8_t> cat;
     std::vector<int32_t> num_of;  // numeric index of a feature, -1 for categorical
     std::vector<void *> allocs;
+    // The staging of one chunk of rows, or (keeps) the whole matrix, which a
+    // context then bins without a second upload (fbh_sketch_rows).
     float *stage = nullptr, *comp = nullptr;
+    bool keeps = false;
+    hipStream_t copy = nullptr;  // keeps: uploads run beside the kernels of earlier rows
+    hipEvent_t arrived = nullptr;
+    RowPipe pipe;
     uint32_t *cnt = nullptr, *off = nullptr, *zero = nullptr, *cat_bad = nullptr;
     int32_t *d_num_of = nullptr, *cat_max = nullptr;
     uint64_t *n_valid = nullptr;
+    std::vector<uint64_t> valid;  // n_valid, once the cuts are taken
     bool finished = false;
 
     template <class T>
@@ -729,9 +803,21 @@ struct fbh_sketch {
         allocs.push_back(p);
         return static_cast<T *>(p);
     }
+    // Frees everything but the kept rows.
+    void trim() {
+        for (void *p : allocs)
+            if (!keeps || p != stage) (void)hipFree(p);
+        allocs.clear();
+        if (keeps) allocs.push_back(stage);
+        pipe.release();
+    }
     ~fbh_sketch() {
         if (stream) (void)hipStreamSynchronize(stream);
+        if (copy) (void)hipStreamSynchronize(copy);
+        pipe.release();
         for (void *p : allocs) (void)hipFree(p);
+        if (arrived) (void)hipEventDestroy(arrived);
+        if (copy) (void)hipStreamDestroy(copy);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -795,7 +881,13 @@ int fbh_sketch_create(int device, uint64_t n_rows, uint32_t n_features, uint32_t
         sk_check(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), "stream creation");
         s->stage_rows = stage_rows_of(n_rows, n_features);
         const uint64_t tiles = (s->stage_rows + SK_ROWS - 1) / SK_ROWS;
-        s->stage = s->alloc<float>(s->stage_rows * n_features, "sketch row staging");
+        s->keeps = n_features && keeps_rows(n_rows, n_features, need, room, memory_budget);
+        if (s->keeps) {
+            sk_check(hipStreamCreateWithFlags(&s->copy, hipStreamNonBlocking), "stream creation");
+            sk_check(hipEventCreateWithFlags(&s->arrived, hipEventDisableTiming), "event");
+        }
+        s->stage = s->alloc<float>((s->keeps ? n_rows : s->stage_rows) * n_features,
+                                   "sketch row staging");
         s->cnt = s->alloc<uint32_t>(tiles * s->n_num, "sketch counts");
         s->off = s->alloc<uint32_t>(tiles * s->n_num, "sketch offsets");
         s->comp = s->alloc<float>(n_rows * s->n_num, "sketch values");
@@ -830,15 +922,27 @@ int fbh_sketch_push_rows(fbh_sketch *s, const float *x, uint64_t n_rows) {
         }
         sk_check(hipSetDevice(s->device), "hipSetDevice");
         const uint64_t nf = s->nf;
-        for (uint64_t r = 0; r < n_rows; r += s->stage_rows) {
-            const uint64_t b = std::min(s->stage_rows, n_rows - r);
-            // Stream order: the copy waits for the previous chunk's kernels.
-            sk_check(hipMemcpyAsync(s->stage, x + r * nf, 4 * b * nf, hipMemcpyHostToDevice,
-                                    s->stream),
-                     "row upload");
+        // Kept rows have their own places, so a chunk's upload runs beside the
+        // kernels of the chunk before; in a staging it waits for them.
+        const uint64_t step = s->keeps ? std::min(s->stage_rows, KEEP_CHUNK_BYTES / (4 * nf) + 1)
+                                       : s->stage_rows;
+        const bool piped = s->keeps && 4 * s->n_rows * nf >= RowPipe::PIPE_LEAST;
+        for (uint64_t r = 0; r < n_rows; r += step) {
+            const uint64_t b = std::min(step, n_rows - r);
+            float *rows = s->keeps ? s->stage + (s->pushed + r) * nf : s->stage;
+            hipStream_t up = s->keeps ? s->copy : s->stream;
+            if (piped)
+                s->pipe.copy(s->device, rows, x + r * nf, 4 * b * nf, up);
+            else
+                sk_check(hipMemcpyAsync(rows, x + r * nf, 4 * b * nf, hipMemcpyHostToDevice, up),
+                         "row upload");
+            if (s->keeps) {
+                sk_check(hipEventRecord(s->arrived, up), "event");
+                sk_check(hipStreamWaitEvent(s->stream, s->arrived, 0), "event");
+            }
             const uint32_t tiles = (uint32_t)((b + SK_ROWS - 1) / SK_ROWS);
             const dim3 grid(tiles, (uint32_t)((nf + SK_FEATS - 1) / SK_FEATS));
-            hipLaunchKernelGGL(sk_count_kernel, grid, dim3(SK_TPB), 0, s->stream, s->stage, b,
+            hipLaunchKernelGGL(sk_count_kernel, grid, dim3(SK_TPB), 0, s->stream, rows, b,
                                (uint32_t)nf, s->d_num_of, s->n_num, s->cnt, s->zero, s->cat_max,
                                s->cat_bad);
             sk_check(hipGetLastError(), "sketch count");
@@ -846,12 +950,13 @@ int fbh_sketch_push_rows(fbh_sketch *s, const float *x, uint64_t n_rows) {
                 hipLaunchKernelGGL(sk_offsets_kernel, dim3(s->n_num), dim3(SK_TPB), 0, s->stream,
                                    s->cnt, tiles, s->n_num, s->off, s->n_valid);
                 sk_check(hipGetLastError(), "sketch offsets");
-                hipLaunchKernelGGL(sk_compact_kernel, grid, dim3(SK_TPB), 0, s->stream, s->stage, b,
+                hipLaunchKernelGGL(sk_compact_kernel, grid, dim3(SK_TPB), 0, s->stream, rows, b,
                                    (uint32_t)nf, s->d_num_of, s->n_num, s->off, s->comp, s->n_rows);
                 sk_check(hipGetLastError(), "sketch compaction");
             }
         }
-        sk_check(hipStreamSynchronize(s->stream), "row sketching");  // the caller may reuse x
+        // the caller may reuse x
+        sk_check(hipStreamSynchronize(s->keeps ? s->copy : s->stream), "row sketching");
         s->pushed += n_rows;
     });
 }
@@ -860,8 +965,9 @@ int fbh_sketch_missing(const fbh_sketch *s, uint64_t *missing) {
     return sk_guard([&] {
         if (!s || !missing) throw SkError(FBH_INPUT_ERROR, "null argument");
         sk_check(hipSetDevice(s->device), "hipSetDevice");
-        std::vector<uint64_t> n_valid(s->n_num);
-        if (s->n_num) {
+        std::vector<uint64_t> n_valid = s->valid;  // once the cuts are taken
+        if (!s->finished && s->n_num) {
+            n_valid.resize(s->n_num);
             sk_check(hipMemcpyAsync(n_valid.data(), s->n_valid, 8ull * s->n_num,
                                     hipMemcpyDeviceToHost, s->stream),
                      "download");
@@ -896,6 +1002,7 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
                                     s->stream), "download");
         }
         sk_check(hipStreamSynchronize(s->stream), "download");
+        s->valid = n_valid;
         for (uint32_t f = 0; f < nf; f++)
             if (s->cat[f] && cat_bad[f])
                 throw SkError(FBH_INPUT_ERROR,
@@ -1077,6 +1184,8 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
             sk_check(hipStreamSynchronize(s->stream), "sketch");
         }
 
+        s->trim();
+
         // ---- the flat cuts ----
         uint64_t total = 0;
         for (uint32_t f = 0; f < nf; f++) {
@@ -1109,6 +1218,10 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
             }
         }
     });
+}
+
+const float *fbh_sketch_rows(const fbh_sketch *s) {
+    return s && s->keeps && s->pushed == s->n_rows ? s->stage : nullptr;
 }
 
 int fbh_sketch_destroy(fbh_sketch *s) {

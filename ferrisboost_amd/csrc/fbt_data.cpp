@@ -262,7 +262,8 @@ Cuts sketch_matrix(const float *x, uint64_t n, uint32_t nf, uint32_t max_bin, co
 
 Cuts sketch_matrix_device(int device, const RowSource &src, uint64_t n, uint32_t nf,
                           uint32_t max_bin, const uint8_t *cat, uint64_t memory_budget,
-                          unsigned threads) {
+                          unsigned threads, fbh_sketch **kept) {
+    *kept = nullptr;
     fbh_sketch *raw = nullptr;
     auto call = [](int rc) {
         if (rc == FBH_OK) return;
@@ -284,7 +285,7 @@ Cuts sketch_matrix_device(int device, const RowSource &src, uint64_t n, uint32_t
     call(fbh_sketch_cuts(s.get(), values.data(), cap, offsets.data(), host.data()));
     std::vector<uint64_t> missing(nf);
     call(fbh_sketch_missing(s.get(), missing.data()));
-    s.reset();
+    if (!fbh_sketch_rows(s.get())) s.reset();
     std::vector<std::vector<float>> per(nf);
     std::vector<uint32_t> on_host;
     for (uint32_t f = 0; f < nf; f++) {
@@ -317,6 +318,7 @@ Cuts sketch_matrix_device(int device, const RowSource &src, uint64_t n, uint32_t
     c.full.assign(nf, 0);
     for (uint32_t f = 0; f < nf; f++)
         if (!c.is_cat(f) && c.n_bins(f) == 256 && missing[f] == 0) c.full[f] = 1;
+    *kept = s.release();
     return c;
 }
 

@@ -11,6 +11,8 @@
 
 #include "fbtrain.h"
 
+struct fbh_sketch;
+
 namespace fbt {
 
 struct InputError : std::runtime_error {
@@ -82,10 +84,11 @@ Cuts sketch_matrix(const float *x, uint64_t n_rows, uint32_t n_features, uint32_
 
 // The same cuts from the device sketch (fbh_sketch_*), for unit row
 // weights; a feature the device leaves to the host (both zero signs) is
-// sketched here.
+// sketched here. *kept (destroy it with fbh_sketch_destroy) is the sketch when it
+// keeps the rows on the device, else null.
 Cuts sketch_matrix_device(int device, const RowSource &src, uint64_t n_rows,
                           uint32_t n_features, uint32_t max_bin, const uint8_t *categorical,
-                          uint64_t memory_budget, unsigned threads);
+                          uint64_t memory_budget, unsigned threads, fbh_sketch **kept);
 
 // Cuts handed in by a caller (fbt_train_cuts): per feature strictly
 // increasing finite values, at most max_bin - 1 for a numeric feature and

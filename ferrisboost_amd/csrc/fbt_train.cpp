@@ -1157,12 +1157,16 @@ Model train(const RowSource &src, uint64_t n, uint32_t nf, const float *y, const
     const bool device_sketch =
         !given && !w && !p.host_sketch &&
         fbh_sketch_fits(p.device, n, nf, p.max_bin, cat, p.gpu_memory_budget);
+    // the sketch, while it keeps the rows on the device for the binning
+    std::unique_ptr<fbh_sketch, int (*)(fbh_sketch *)> on_device(nullptr, fbh_sketch_destroy);
     if (given) {
         check_cuts(*given, nf, p.max_bin, cat);
         m.cuts = *given;
     } else if (device_sketch) {
+        fbh_sketch *kept = nullptr;
         m.cuts = sketch_matrix_device(p.device, src, n, nf, p.max_bin, cat, p.gpu_memory_budget,
-                                      threads);
+                                      threads, &kept);
+        on_device.reset(kept);
     } else {
         materialise();
         m.cuts = sketch_matrix(x, n, nf, p.max_bin, w, cat, threads);
@@ -1279,13 +1283,17 @@ Model train(const RowSource &src, uint64_t n, uint32_t nf, const float *y, const
     if (device_binning) {
         call(fbh_set_cuts(ctx.get(), m.cuts.values.data(), m.cuts.offsets.data(),
                           m.cuts.categorical.data()));
-        RowSource rows = src;
-        rows.x = x;
-        rows.each_chunk(n, nf, [&](uint64_t r0, uint64_t k, const float *chunk) {
-            const uint64_t step = 1u << 20;
-            for (uint64_t b = 0; b < k; b += step)
-                call(fbh_upload_rows(ctx.get(), chunk + b * nf, r0 + b, std::min(step, k - b)));
-        });
+        if (on_device) {
+            call(fbh_bin_rows(ctx.get(), fbh_sketch_rows(on_device.get()), 0, n));
+        } else {
+            RowSource rows = src;
+            rows.x = x;
+            rows.each_chunk(n, nf, [&](uint64_t r0, uint64_t k, const float *chunk) {
+                const uint64_t step = 1u << 20;
+                for (uint64_t b = 0; b < k; b += step)
+                    call(fbh_upload_rows(ctx.get(), chunk + b * nf, r0 + b, std::min(step, k - b)));
+            });
+        }
         call(fbh_finish_rows(ctx.get()));
     } else {
         materialise();
@@ -1296,6 +1304,7 @@ Model train(const RowSource &src, uint64_t n, uint32_t nf, const float *y, const
             call(fbh_upload_block(ctx.get(), feats.data(), (uint32_t)feats.size(), wdt, buf.data()));
         }
     }
+    on_device.reset();
     const double bin_s = std::chrono::duration<double>(Clock::now() - t_bin).count();
     g_stats = fbt_stats{};
     g_stats.device_binning = device_binning ? 1 : 0;

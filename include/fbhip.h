@@ -212,6 +212,9 @@ uint64_t fbh_rows_staging_bytes(const fbh_ctx *ctx);
 /* Rows [row0, row0 + n_rows) of the matrix, row-major with the context's
  * n_features columns (x points at row row0). */
 int fbh_upload_rows(fbh_ctx *ctx, const float *x, uint64_t row0, uint64_t n_rows);
+/* fbh_upload_rows of rows that are in device memory already (x points at row
+ * row0 there, complete when the call is made). */
+int fbh_bin_rows(fbh_ctx *ctx, const float *x, uint64_t row0, uint64_t n_rows);
 /* Every feature's tile records from its binned column; the features count
  * as uploaded from then on. */
 int fbh_finish_rows(fbh_ctx *ctx);
@@ -264,6 +267,12 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
  * trainer stores a 256-bin numeric feature with none in 8-bit cells. Has no
  * counterpart in the reference (whose bins are 32-bit). */
 int fbh_sketch_missing(const fbh_sketch *s, uint64_t *missing);
+/* The rows pushed, row-major on the device, once all of the created row count
+ * are: a sketch created without a memory budget keeps them while free HBM holds
+ * the sketch and four times the matrix (they come on top of
+ * fbh_sketch_device_bytes). NULL otherwise. They stay until fbh_sketch_destroy;
+ * fbh_bin_rows bins them without a second upload. */
+const float *fbh_sketch_rows(const fbh_sketch *s);
 int fbh_sketch_destroy(fbh_sketch *s);
 
 /* ------------------------------------------------------------ gradients */
