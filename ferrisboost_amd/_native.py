@@ -346,8 +346,7 @@ def hip() -> C.CDLL:
                                             P, C.c_uint32, C.c_uint32, C.c_float, C.POINTER(P)]
         L.fbh_shap_model_destroy.argtypes = [P]
         L.fbh_shap_set_host_order.argtypes = [P, C.c_int]
-        L.fbh_sketch_rows.argtypes = [P]
-        L.fbh_sketch_rows.restype = P
+        L.fbh_sketch_rows.argtypes = [P, C.POINTER(P)]
         L.fbh_bin_rows.argtypes = [P, P, C.c_uint64, C.c_uint64]
         L.fbh_shap_contribs.argtypes = [P, P, C.c_uint64, P, P]
         L.fbh_shap_contribs_device.argtypes = [P, P, C.c_uint64, P, P, C.c_int]

@@ -1220,8 +1220,11 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
     });
 }
 
-const float *fbh_sketch_rows(const fbh_sketch *s) {
-    return s && s->keeps && s->pushed == s->n_rows ? s->stage : nullptr;
+int fbh_sketch_rows(const fbh_sketch *s, const float **rows) {
+    return sk_guard([&] {
+        if (!s || !rows) throw SkError(FBH_INPUT_ERROR, "null argument");
+        *rows = s->keeps && s->pushed == s->n_rows ? s->stage : nullptr;
+    });
 }
 
 int fbh_sketch_destroy(fbh_sketch *s) {

@@ -285,7 +285,9 @@ Cuts sketch_matrix_device(int device, const RowSource &src, uint64_t n, uint32_t
     call(fbh_sketch_cuts(s.get(), values.data(), cap, offsets.data(), host.data()));
     std::vector<uint64_t> missing(nf);
     call(fbh_sketch_missing(s.get(), missing.data()));
-    if (!fbh_sketch_rows(s.get())) s.reset();
+    const float *rows = nullptr;
+    call(fbh_sketch_rows(s.get(), &rows));
+    if (!rows) s.reset();
     std::vector<std::vector<float>> per(nf);
     std::vector<uint32_t> on_host;
     for (uint32_t f = 0; f < nf; f++) {

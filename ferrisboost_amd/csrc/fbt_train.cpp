@@ -1284,7 +1284,9 @@ Model train(const RowSource &src, uint64_t n, uint32_t nf, const float *y, const
         call(fbh_set_cuts(ctx.get(), m.cuts.values.data(), m.cuts.offsets.data(),
                           m.cuts.categorical.data()));
         if (on_device) {
-            call(fbh_bin_rows(ctx.get(), fbh_sketch_rows(on_device.get()), 0, n));
+            const float *rows = nullptr;
+            call(fbh_sketch_rows(on_device.get(), &rows));
+            call(fbh_bin_rows(ctx.get(), rows, 0, n));
         } else {
             RowSource rows = src;
             rows.x = x;

@@ -270,9 +270,9 @@ int fbh_sketch_missing(const fbh_sketch *s, uint64_t *missing);
 /* The rows pushed, row-major on the device, once all of the created row count
  * are: a sketch created without a memory budget keeps them while free HBM holds
  * the sketch and four times the matrix (they come on top of
- * fbh_sketch_device_bytes). NULL otherwise. They stay until fbh_sketch_destroy;
+ * fbh_sketch_device_bytes). *rows is NULL otherwise. They stay until fbh_sketch_destroy;
  * fbh_bin_rows bins them without a second upload. */
-const float *fbh_sketch_rows(const fbh_sketch *s);
+int fbh_sketch_rows(const fbh_sketch *s, const float **rows);
 int fbh_sketch_destroy(fbh_sketch *s);
 
 /* ------------------------------------------------------------ gradients */
