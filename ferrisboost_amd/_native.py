@@ -236,7 +236,7 @@ HIP_SYMBOLS = [
     "fbh_hist_timing", "fbh_set_timing", "fbh_build_histogram", "fbh_partition_rows",
     "fbh_shap_model_create", "fbh_shap_model_destroy", "fbh_shap_contribs",
     "fbh_shap_contribs_device", "fbh_shap_last_ms", "fbh_shap_interactions",
-    "fbh_shap_set_host_order",
+    "fbh_shap_set_host_order", "fbh_release_cached",
     "fbh_saabas_contribs", "fbh_predict", "fbh_predict_device", "fbh_shap_contribs_noalloc",
 ]
 TRAIN_SYMBOLS = [
@@ -346,6 +346,7 @@ def hip() -> C.CDLL:
                                             P, C.c_uint32, C.c_uint32, C.c_float, C.POINTER(P)]
         L.fbh_shap_model_destroy.argtypes = [P]
         L.fbh_shap_set_host_order.argtypes = [P, C.c_int]
+        L.fbh_release_cached.argtypes = [C.c_int]
         L.fbh_sketch_rows.argtypes = [P, C.POINTER(P)]
         L.fbh_bin_rows.argtypes = [P, P, C.c_uint64, C.c_uint64]
         L.fbh_shap_contribs.argtypes = [P, P, C.c_uint64, P, P]

@@ -474,35 +474,36 @@ struct fbh_ctx {
     double hist_ms = 0.0;
     uint64_t hist_launches = 0, hist_bytes = 0;
 
+    bool keep = true;  // what is given back is kept for the next context (fbhip_keep.hip)
+
     ~fbh_ctx() { release(); }
 
     void release() {
         q_forget(-1);  // the sums read pin_q and wait on chunk_ev
         if (device >= 0) (void)hipSetDevice(device);
+        // Nothing may be in flight on what is given back.
         if (stream) (void)hipStreamSynchronize(stream);
-        for (auto &a : allocs)
-            if (a.p) (void)hipFree(a.p);
+        if (copy_stream) (void)hipStreamSynchronize(copy_stream);
+        if (up_stream) (void)hipStreamSynchronize(up_stream);
+        for (auto &a : allocs) keep_free(KeepKind::device, a.p, keep);
         allocs.clear();
         for (int k = 0; k < STAGE_SLOTS; k++) {
-            if (pin_stage[k].p) (void)hipHostFree(pin_stage[k].p);
+            keep_free(KeepKind::host_coherent, pin_stage[k].p, keep);
             pin_stage[k].p = nullptr;
             if (stage_ev[k]) (void)hipEventDestroy(stage_ev[k]);
             stage_ev[k] = nullptr;
         }
-        if (pin_leaves.p) (void)hipHostFree(pin_leaves.p);
-        if (pin_out.p) (void)hipHostFree(pin_out.p);
         for (int k = 0; k < 2; k++) {
-            if (grow.out[k].p) (void)hipHostFree(grow.out[k].p);
+            keep_free(KeepKind::host_coherent, grow.out[k].p, keep);
             grow.out[k].p = nullptr;
             if (grow.done[k]) (void)hipEventDestroy(grow.done[k]);
             grow.done[k] = nullptr;
         }
-        if (pin_ids.p) (void)hipHostFree(pin_ids.p);
-        if (pin_src.p) (void)hipHostFree(pin_src.p);
-        if (pin_q.p) (void)hipHostFree(pin_q.p);
-        pin_leaves.p = pin_out.p = pin_ids.p = pin_src.p = pin_q.p = nullptr;
+        for (PinnedBuf *b : {&pin_leaves, &pin_out, &pin_ids, &pin_src, &pin_q}) {
+            keep_free(KeepKind::host, b->p, keep);
+            b->p = nullptr;
+        }
         q_terms = nullptr;
-        if (copy_stream) (void)hipStreamSynchronize(copy_stream);
         for (void *h : host_allocs) (void)hipHostFree(h);
         host_allocs.clear();
         for (int k = 0; k < 4; k++) {
@@ -510,15 +511,10 @@ struct fbh_ctx {
             if (win_free[k]) (void)hipEventDestroy(win_free[k]);
             win_ready[k] = win_free[k] = nullptr;
         }
-        if (copy_stream) (void)hipStreamDestroy(copy_stream);
-        copy_stream = nullptr;
-        if (up_stream) (void)hipStreamSynchronize(up_stream);
         for (auto e : chunk_ev) (void)hipEventDestroy(e);
         chunk_ev.clear();
         if (up_done) (void)hipEventDestroy(up_done);
         up_done = nullptr;
-        if (up_stream) (void)hipStreamDestroy(up_stream);
-        up_stream = nullptr;
         for (auto &e : ev_pool) {
             (void)hipEventDestroy(e.first);
             (void)hipEventDestroy(e.second);
@@ -526,15 +522,17 @@ struct fbh_ctx {
         ev_pool.clear();
         if (leaves_done) (void)hipEventDestroy(leaves_done);
         leaves_done = nullptr;
-        if (stream) (void)hipStreamDestroy(stream);
-        stream = nullptr;
+        for (hipStream_t *s : {&copy_stream, &up_stream, &stream}) {
+            keep_stream_back(device, *s);
+            *s = nullptr;
+        }
     }
 
     template <class T>
     T *alloc(size_t count, const char *what) {
         size_t bytes = std::max<size_t>(count * sizeof(T), 256);
         void *p = nullptr;
-        hipError_t e = hipMalloc(&p, bytes);
+        hipError_t e = keep_alloc(KeepKind::device, &p, bytes);
         if (e != hipSuccess)
             throw RuntimeError(std::string("device allocation of ") + what + " (" +
                                std::to_string(bytes) + " bytes) failed: " + hipGetErrorString(e));
@@ -549,7 +547,7 @@ struct fbh_ctx {
         sync();
         for (size_t i = 0; i < allocs.size(); i++)
             if (allocs[i].p == p) {
-                (void)hipFree(p);
+                keep_free(KeepKind::device, p, keep);
                 device_bytes -= allocs[i].bytes;
                 allocs.erase(allocs.begin() + (long)i);
                 return;
@@ -563,7 +561,7 @@ struct fbh_ctx {
     int64_t *partial_buffer(uint64_t bytes);
 
     void pinned(PinnedBuf &b, size_t bytes) {
-        check(hipHostMalloc(&b.p, bytes, hipHostMallocDefault), "pinned host allocation");
+        check(keep_alloc(KeepKind::host, &b.p, bytes), "pinned host allocation");
         b.bytes = bytes;
     }
     // Coherent pinned memory that kernels read through its device view:
@@ -571,7 +569,7 @@ struct fbh_ctx {
     // (send_mapped) instead of a copy-engine transfer, whose handoff between
     // engines stalls the queue for tens of microseconds.
     void pinned_mapped(PinnedBuf &b, size_t bytes) {
-        check(hipHostMalloc(&b.p, bytes, hipHostMallocCoherent), "pinned host allocation");
+        check(keep_alloc(KeepKind::host_coherent, &b.p, bytes), "pinned host allocation");
         b.bytes = bytes;
         check(hipHostGetDevicePointer(&b.dev, b.p, 0), "device view of pinned memory");
     }
@@ -1203,7 +1201,10 @@ int fbh_ctx_create(int device, uint64_t n_rows, const fbh_shape *shape, const fb
             throw InputError("device " + std::to_string(device) + " does not exist");
         c->device = device;
         check(hipSetDevice(device), "hipSetDevice");
-        check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "stream creation");
+        // With a memory budget nothing is held beside the context.
+        c->keep = conf.memory_budget == 0;
+        if (!c->keep) (void)keep_release(device);
+        check(keep_stream(&c->stream), "stream creation");
         {
             hipDeviceProp_t prop;
             check(hipGetDeviceProperties(&prop, device), "hipGetDeviceProperties");
@@ -1211,7 +1212,8 @@ int fbh_ctx_create(int device, uint64_t n_rows, const fbh_shape *shape, const fb
         }
         size_t free_b = 0, total_b = 0;
         check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-        c->plan = plan_layout(*c, budget_of(conf, free_b));
+        // what is kept goes when it is in the way of an allocation
+        c->plan = plan_layout(*c, budget_of(conf, free_b + keep_bytes(device)));
         const fbh_plan &P = c->plan;
 
         // ---- allocation, once, as planned ----
@@ -1253,7 +1255,7 @@ int fbh_ctx_create(int device, uint64_t n_rows, const fbh_shape *shape, const fb
                 if (!t.resident)
                     for (uint32_t f : t.feats)
                         c->host_cols[f] = c->host_alloc(n_rows * c->width[f], "streamed column");
-            check(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking), "stream creation");
+            check(keep_stream(&c->copy_stream), "stream creation");
             for (int k = 0; k < 4; k++) {
                 check(hipEventCreateWithFlags(&c->win_ready[k], hipEventDisableTiming), "event");
                 check(hipEventCreateWithFlags(&c->win_free[k], hipEventDisableTiming), "event");
@@ -1872,7 +1874,7 @@ int fbh_set_objective(fbh_ctx *c, uint32_t objective, const float *labels,
             c->sig = c->alloc<float>(c->n_rows, "sigmoids");
             c->pinned(c->pin_ids, std::max<uint64_t>(2 * c->n_rows, 64));
             c->pinned(c->pin_src, std::max<uint64_t>(4 * c->n_rows, 64));
-            check(hipStreamCreateWithFlags(&c->up_stream, hipStreamNonBlocking), "stream");
+            check(keep_stream(&c->up_stream), "stream");
             check(hipEventCreateWithFlags(&c->up_done, hipEventDisableTiming), "event");
             for (int k = 0; k < EXCHANGE_CHUNKS; k++) {
                 hipEvent_t e;
@@ -3321,12 +3323,12 @@ void ensure_grow(fbh_ctx *c, uint32_t D) {
     G.leaves = c->alloc<LeafDev>(G.leaf_cap, "grown tree leaves");
     G.leaf_vals = c->alloc<float>(G.leaf_cap, "grown tree leaf values");
     for (int k = 0; k < 2; k++) {
-        if (G.out[k].p) (void)hipHostFree(G.out[k].p);
+        keep_free(KeepKind::host_coherent, G.out[k].p, c->keep);
         G.out[k].p = nullptr;
         // Coherent: the kernel's writes go to host memory, not the device caches.
         const size_t bytes = al256(sizeof(GrowState)) + al256(sizeof(TreeNodeDev) * G.tree_cap) +
                              al256(8 * G.cat_cap) + al256(4 * G.leaf_cap);
-        check(hipHostMalloc(&G.out[k].p, bytes, hipHostMallocCoherent), "pinned host allocation");
+        check(keep_alloc(KeepKind::host_coherent, &G.out[k].p, bytes), "pinned host allocation");
         G.out[k].bytes = bytes;
         void *dv = nullptr;
         check(hipHostGetDevicePointer(&dv, G.out[k].p, 0), "device view of the tree buffer");
@@ -3838,8 +3840,12 @@ int fbh_sigmoid_device(int device, const float *in, uint64_t n, float *out) {
         if (n == 0) return;
         check(hipSetDevice(device), "hipSetDevice");
         float *d = nullptr;
-        check(hipMalloc(&d, 8 * n), "device allocation");
-        std::unique_ptr<float, hipError_t (*)(void *)> own(d, hipFree);
+        check(keep_alloc(KeepKind::device, reinterpret_cast<void **>(&d), 8 * n), "device allocation");
+        const auto give_back = [](void *p) {
+            (void)hipStreamSynchronize(nullptr);
+            keep_free(KeepKind::device, p);
+        };
+        std::unique_ptr<float, decltype(give_back)> own(d, give_back);
         check(hipMemcpy(d, in, 4 * n, hipMemcpyHostToDevice), "input upload");
         check(launch_sigmoid(d, n, d + n, nullptr), "sigmoid");
         check(hipMemcpy(out, d + n, 4 * n, hipMemcpyDeviceToHost), "output download");

@@ -7,6 +7,17 @@
 
 namespace fbh {
 
+// Memory and streams that jobs take and give back (fbhip_keep.hip). Calls act on
+// the current device. All work on a block must have completed when it is given
+// back; a block given back without `keep` goes at once.
+enum class KeepKind { device, host, host_coherent };
+hipError_t keep_alloc(KeepKind kind, void **p, uint64_t bytes);
+void keep_free(KeepKind kind, void *p, bool keep = true) noexcept;
+bool keep_release(int device) noexcept;     // frees what is kept; whether there was any
+uint64_t keep_bytes(int device) noexcept;   // device memory kept
+hipError_t keep_stream(hipStream_t *s);     // a non-blocking stream
+void keep_stream_back(int device, hipStream_t s) noexcept;  // waits for it
+
 constexpr int HIST_TPB = 256;      // threads of one histogram workgroup
 constexpr int SPLIT_TPB = 256;     // threads of one split-scan workgroup
 constexpr int PART_TPB = 256;      // threads of one partition workgroup

@@ -781,13 +781,13 @@ struct fbh_shap_model {
     ~fbh_shap_model() {
         if (device >= 0) (void)hipSetDevice(device);
         if (stream) (void)hipStreamSynchronize(stream);
-        for (void *p : allocs) (void)hipFree(p);
-        if (work) (void)hipFree(work);
-        if (staging) (void)hipFree(staging);
-        if (pinned) (void)hipHostFree(pinned);
+        for (void *p : allocs) keep_free(KeepKind::device, p);
+        keep_free(KeepKind::device, work);
+        keep_free(KeepKind::device, staging);
+        keep_free(KeepKind::host, pinned);
         if (e0) (void)hipEventDestroy(e0);
         if (e1) (void)hipEventDestroy(e1);
-        if (stream) (void)hipStreamDestroy(stream);
+        keep_stream_back(device, stream);
     }
     // The arrays added so far, laid out in one allocation and sent in one copy.
     struct Arrays {
@@ -803,7 +803,7 @@ struct fbh_shap_model {
     };
     void upload(const Arrays &a) {
         void *p = nullptr;
-        chk(hipMalloc(&p, a.bytes.size()), "model arrays");
+        chk(keep_alloc(KeepKind::device, &p, a.bytes.size()), "model arrays");
         allocs.push_back(p);
         chk(hipMemcpy(p, a.bytes.data(), a.bytes.size(), hipMemcpyHostToDevice), "model arrays");
         for (const auto &f : a.place) f(static_cast<unsigned char *>(p));
@@ -1066,12 +1066,12 @@ bool grow_work(fbh_shap_model *m, uint64_t want, uint64_t least) {
     if (m->work_bytes >= want) return true;
     if (m->work) {
         chk(hipStreamSynchronize(m->stream), "workspace");
-        chk(hipFree(m->work), "workspace");
+        keep_free(KeepKind::device, m->work);
     }
     m->work = nullptr;
     m->work_bytes = 0;
     for (uint64_t b = want; b >= least && !m->work; b /= 2)
-        if (hipMalloc(&m->work, b) == hipSuccess) m->work_bytes = b;
+        if (keep_alloc(KeepKind::device, &m->work, b) == hipSuccess) m->work_bytes = b;
         else (void)hipGetLastError();
     return m->work != nullptr;
 }
@@ -1283,7 +1283,7 @@ void run_host_alloc(fbh_shap_model *m, Kind k, const float *rows, uint64_t n_row
     const uint64_t per_row = 4ull * (nf + 1 + w);
     std::unique_lock<std::mutex> mine(m->host_mu, std::try_to_lock);
     if (mine && n_rows <= PINNED_BYTES / per_row && runs_in_place(m, k)) {
-        if (!m->pinned) chk(hipHostMalloc(&m->pinned, PINNED_BYTES + 1024, hipHostMallocDefault), "pinned");
+        if (!m->pinned) chk(keep_alloc(KeepKind::host, &m->pinned, PINNED_BYTES + 1024), "pinned");
         float *x = static_cast<float *>(m->pinned);
         float *mg = x + round256(4 * n_rows * nf) / 4, *o = mg + round256(4 * n_rows) / 4;
         std::memcpy(x, rows, 4 * n_rows * nf);
@@ -1303,20 +1303,26 @@ void run_host_alloc(fbh_shap_model *m, Kind k, const float *rows, uint64_t n_row
     const uint64_t o_rows = round256(4 * st.cap_rows * nf);
     const uint64_t o_out = o_rows + round256(4 * st.cap_rows);
     const uint64_t need = o_out + 4 * st.cap_rows * w + 4;
-    std::unique_ptr<void, decltype(&hipFree)> own(nullptr, hipFree);
+    // A call's own staging goes back once the stream is done with it.
+    auto give_back = [m](void *p) {
+        (void)hipStreamSynchronize(m->stream);
+        keep_free(KeepKind::device, p);
+    };
+    std::unique_ptr<void, decltype(give_back)> own(nullptr, give_back);
     unsigned char *base;
     if (mine && need <= KEEP_STAGING) {
         if (m->staging_bytes < need) {
-            if (m->staging) chk(hipFree(m->staging), "staging");
+            chk(hipStreamSynchronize(m->stream), "staging");
+            keep_free(KeepKind::device, m->staging);
             m->staging = nullptr;
             m->staging_bytes = 0;
-            chk(hipMalloc(&m->staging, need), "staging");
+            chk(keep_alloc(KeepKind::device, &m->staging, need), "staging");
             m->staging_bytes = need;
         }
         base = static_cast<unsigned char *>(m->staging);
     } else {
         void *p = nullptr;
-        chk(hipMalloc(&p, need), "staging");
+        chk(keep_alloc(KeepKind::device, &p, need), "staging");
         own.reset(p);
         base = static_cast<unsigned char *>(p);
     }
@@ -1368,7 +1374,7 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         auto m = std::make_unique<fbh_shap_model>();
         m->device = device;
         chk(hipSetDevice(device), "hipSetDevice");
-        chk(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "stream");
+        chk(keep_stream(&m->stream), "stream");
         chk(hipEventCreate(&m->e0), "event");
         chk(hipEventCreate(&m->e1), "event");
         const uint32_t total = tree_offsets[n_trees];

@@ -693,6 +693,7 @@ uint64_t room_of(int device, uint64_t budget) {
     size_t free_b = 0, total_b = 0;
     if (hipSetDevice(device) != hipSuccess || hipMemGetInfo(&free_b, &total_b) != hipSuccess)
         return 0;
+    free_b += keep_bytes(device);  // goes when it is in the way of an allocation
     const uint64_t reserve = std::max<uint64_t>(free_b / 100 * 15, 512ull << 20);
     return free_b > reserve ? free_b - reserve : 0;
 }
@@ -724,7 +725,7 @@ struct RowPipe {
     void copy(int device, void *dst, const void *src, uint64_t bytes, hipStream_t s) {
         if (!pinned) {
             void *p = nullptr;
-            sk_check(hipHostMalloc(&p, THREADS * SLOTS * PIECE, hipHostMallocDefault), "row pipe");
+            sk_check(keep_alloc(KeepKind::host, &p, THREADS * SLOTS * PIECE), "row pipe");
             pinned = static_cast<unsigned char *>(p);
             for (auto &t : done)
                 for (hipEvent_t &e : t)
@@ -760,7 +761,7 @@ struct RowPipe {
                 if (e) (void)hipEventDestroy(e);
                 e = nullptr;
             }
-        if (pinned) (void)hipHostFree(pinned);
+        keep_free(KeepKind::host, pinned);
         pinned = nullptr;
     }
 };
@@ -795,18 +796,21 @@ struct fbh_sketch {
     uint64_t *n_valid = nullptr;
     std::vector<uint64_t> valid;  // n_valid, once the cuts are taken
     bool finished = false;
+    bool keep = true;  // what is given back is kept (fbhip_keep.hip)
 
     template <class T>
     T *alloc(uint64_t count, const char *what) {
         void *p = nullptr;
-        sk_check(hipMalloc(&p, std::max<uint64_t>(count * sizeof(T), 64)), what);
+        sk_check(keep_alloc(KeepKind::device, &p, std::max<uint64_t>(count * sizeof(T), 64)), what);
         allocs.push_back(p);
         return static_cast<T *>(p);
     }
-    // Frees everything but the kept rows.
+    // Frees everything but the kept rows, once the streams are done.
     void trim() {
+        sk_check(hipStreamSynchronize(stream), "sketch");
+        if (copy) sk_check(hipStreamSynchronize(copy), "sketch");
         for (void *p : allocs)
-            if (!keeps || p != stage) (void)hipFree(p);
+            if (!keeps || p != stage) keep_free(KeepKind::device, p, keep);
         allocs.clear();
         if (keeps) allocs.push_back(stage);
         pipe.release();
@@ -815,10 +819,10 @@ struct fbh_sketch {
         if (stream) (void)hipStreamSynchronize(stream);
         if (copy) (void)hipStreamSynchronize(copy);
         pipe.release();
-        for (void *p : allocs) (void)hipFree(p);
+        for (void *p : allocs) keep_free(KeepKind::device, p, keep);
         if (arrived) (void)hipEventDestroy(arrived);
-        if (copy) (void)hipStreamDestroy(copy);
-        if (stream) (void)hipStreamDestroy(stream);
+        keep_stream_back(device, copy);
+        keep_stream_back(device, stream);
     }
 };
 
@@ -878,12 +882,14 @@ int fbh_sketch_create(int device, uint64_t n_rows, uint32_t n_features, uint32_t
             if (!s->cat[f]) s->num_of[f] = (int32_t)s->n_num++;
         }
         sk_check(hipSetDevice(device), "hipSetDevice");
-        sk_check(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), "stream creation");
+        s->keep = memory_budget == 0;
+        if (!s->keep) (void)keep_release(device);
+        sk_check(keep_stream(&s->stream), "stream creation");
         s->stage_rows = stage_rows_of(n_rows, n_features);
         const uint64_t tiles = (s->stage_rows + SK_ROWS - 1) / SK_ROWS;
         s->keeps = n_features && keeps_rows(n_rows, n_features, need, room, memory_budget);
         if (s->keeps) {
-            sk_check(hipStreamCreateWithFlags(&s->copy, hipStreamNonBlocking), "stream creation");
+            sk_check(keep_stream(&s->copy), "stream creation");
             sk_check(hipEventCreateWithFlags(&s->arrived, hipEventDisableTiming), "event");
         }
         s->stage = s->alloc<float>((s->keeps ? n_rows : s->stage_rows) * n_features,

@@ -134,6 +134,11 @@ typedef struct {
 size_t fbh_last_error(char *buf, size_t len);
 /* 1 when a usable gfx950 device is present, 0 otherwise (never errors). */
 int fbh_device_available(int device);
+/* Contexts, sketches and models without a memory budget leave their buffers and
+ * streams to the next one: at most a sixteenth of the device's memory, given back
+ * when an allocation needs it, when something is made with a budget, or here.
+ * Nothing in use is touched. No reference counterpart. */
+int fbh_release_cached(int device);
 
 /* ------------------------------------------------------------ lifecycle */
 /* GpuTrainCtx::new_with_shape (src/backend/cuda/train_ctx.rs:728-1769):
