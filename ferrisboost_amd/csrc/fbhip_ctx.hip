@@ -299,7 +299,11 @@ struct fbh_ctx {
     bool rows_identity = false;
     double *red_f64 = nullptr;
     int64_t *red_i64 = nullptr;
-    uint32_t n_red_blocks = 8192;  // blocks of the bounds and quantisation passes
+    // Blocks of the bounds and quantisation passes, whose results reduce_max_kernel and
+    // grow_prep_kernel go through on one workgroup: a row a thread, and rows in turn
+    // from 8192 blocks on. With 8192 at any size the four kernels took 40 us a tree of
+    // 5000 rows, now 16.
+    uint32_t n_red_blocks = 8192;
 
     // launch tables (device) and their pinned staging
     TileDev *d_tiles = nullptr;
@@ -1101,6 +1105,7 @@ fbh_config configure(fbh_ctx &c, uint64_t n_rows, const fbh_shape *shape, const 
         throw InputError("training data has " + std::to_string(n_rows) +
                          " rows, above the supported limit 4294967295");
     c.n_rows = n_rows;
+    c.n_red_blocks = (uint32_t)std::min<uint64_t>((n_rows + 255) / 256, 8192);
     c.n_features = shape->n_features;
     c.width.assign(shape->width, shape->width + shape->n_features);
     c.n_bins.assign(shape->n_bins, shape->n_bins + shape->n_features);
