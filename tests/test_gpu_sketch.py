@@ -108,6 +108,15 @@ def test_device_sketch_equals_host_sketch(N, max_bin, n):
     _same(N, _mixed(n, n + max_bin), max_bin)
 
 
+@pytest.mark.parametrize("max_bin", [4, 5, 8, 9, 32, 33, 64, 65, 128, 129, 257, 512, 513])
+def test_batch_sizes_on_both_sides_of_the_sorts_blocks(N, max_bin):
+    """Batches of 16 max_bin values are sorted by blocks of 64 to 16384 keys: batches
+    that fill a block, need the next one, lack a value and have one to spare."""
+    limit = 16 * max_bin
+    for n in (limit - 1, limit, 2 * limit + 1):
+        _same(N, _mixed(n, n + max_bin), max_bin)
+
+
 @pytest.mark.parametrize("max_bin", [4, 255])
 def test_many_batches_and_uneven_pushes(N, max_bin):
     """max_bin 4 puts 64 values in a batch: 300k rows make 4688 batches, 13
