@@ -422,10 +422,10 @@ __device__ __forceinline__ float sk_target(float total, uint32_t k, uint32_t slo
 }
 
 // The largest k in [0, slots - 1] with target_k <= m (0: none). The targets
-// never decrease in k, so an estimate from the exact quotient is moved to
+// never decrease in k, so an estimate (`per` is about slots / total) is moved to
 // the boundary by evaluating the targets themselves.
-__device__ uint32_t sk_targets_upto(float m, float total, uint32_t slots) {
-    const double e = (double)m * (double)slots / (double)total;
+__device__ uint32_t sk_targets_upto(float m, float total, uint32_t slots, double per) {
+    const double e = (double)m * per;
     uint32_t k = e <= 0.0 ? 0u : (e >= (double)(slots - 1) ? slots - 1 : (uint32_t)e);
     while (k + 1 <= slots - 1 && sk_target(total, k + 1, slots) <= m) k++;
     while (k >= 1 && sk_target(total, k, slots) > m) k--;
@@ -452,10 +452,23 @@ __device__ void sk_compress_plan(const SkEntry *s, uint32_t n, uint32_t slots, I
     const float total = s[n - 1].rmax;
     for (uint32_t k = 1 + threadIdx.x; k < slots; k += SK_TPB) sel[k] = (IDX)(n - 1);
     __syncthreads();
-    for (uint32_t i = 1 + threadIdx.x; i + 1 < n; i += SK_TPB) {
-        const uint32_t ci = sk_targets_upto(sk_mid(s + i), total, slots);
-        const uint32_t cp = i == 1 ? 0u : sk_targets_upto(sk_mid(s + i - 1), total, slots);
-        for (uint32_t k = cp + 1; k <= ci; k++) sel[k] = (IDX)i;
+    // A wave takes a stretch of the entries, 64 at a time, and passes the last c_i on:
+    // each is found once, without the quotient's division: merges of 400k x
+    // 2000 at 256 bins 35.4 -> 30.5 ms, 10.5M x 28 14.4 -> 12.4.
+    const double per_rank = (double)slots / (double)total;
+    const uint32_t lane = threadIdx.x & 63u, waves = SK_TPB / 64;
+    const uint32_t stretch = (n - 2 + 64 * waves - 1) / (64 * waves) * 64;
+    const uint32_t i0 = 1 + (threadIdx.x >> 6) * stretch, i1 = min(n - 1, i0 + stretch);
+    uint32_t before = 0;
+    if (i0 > 1 && i0 < i1) before = sk_targets_upto(sk_mid(s + i0 - 1), total, slots, per_rank);
+    for (uint32_t b = i0; b < i1; b += 64) {
+        const uint32_t i = b + lane;
+        const uint32_t ci = i < i1 ? sk_targets_upto(sk_mid(s + i), total, slots, per_rank) : 0u;
+        uint32_t cp = __shfl_up(ci, 1, 64);
+        if (lane == 0) cp = before;
+        before = __shfl(ci, 63, 64);
+        if (i < i1)
+            for (uint32_t k = cp + 1; k <= ci; k++) sel[k] = (IDX)i;
     }
     __syncthreads();
     const uint32_t nk = slots - 1;
