@@ -117,6 +117,18 @@ def test_batch_sizes_on_both_sides_of_the_sorts_blocks(N, max_bin):
         _same(N, _mixed(n, n + max_bin), max_bin)
 
 
+def test_feature_groups(N):
+    """More summaries than one group of features holds (2 GiB): the groups share their
+    buffers, with missing values and a feature without any at a group's edge."""
+    n, nf = 250_003, 800
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((n, nf), dtype=np.float32)
+    x[:, ::7] = np.round(x[:, ::7] * 20) + 0.0
+    x[rng.random(n) < 0.3, 5::11] = np.nan
+    x[:, [0, 536, 537, nf - 1]] = np.nan
+    _same(N, x, 16)
+
+
 @pytest.mark.parametrize("max_bin", [4, 255])
 def test_many_batches_and_uneven_pushes(N, max_bin):
     """max_bin 4 puts 64 values in a batch: 300k rows make 4688 batches, 13
