@@ -98,7 +98,8 @@ constexpr uint64_t KEEP_CHUNK_BYTES = 64ull << 20;     // rows uploaded, then sk
 // batch summaries but no fewer than GROUP_FEATS features: a merge of each still gives
 // every CU a workgroup at the counter's last levels. 400k x 2000 at 256 bins takes 33
 // GB in one group, more than is kept for the next job (fbhip_keep.hip), and 11 in groups:
-// the whole job, 40 rounds, 238 -> 226 ms.
+// the whole job, 40 rounds, 239 -> 226 ms, and 221 with a group's task tables
+// built while the groups before it run.
 constexpr uint32_t GROUP_FEATS = 256;
 constexpr uint64_t GROUP_BYTES = 2ull << 30;
 
@@ -1120,9 +1121,6 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
         if (abase[nn]) {
             struct Group {
                 uint32_t j0, j1;
-                std::vector<uint64_t> level_end;  // merges of levels 0..l end at level_end[l]
-                std::vector<std::vector<SkMergeTask>> finals;
-                std::vector<uint64_t> o_final;
             };
             std::vector<Group> groups;
             uint64_t na = 0, nb = 0, nt = 0;  // the largest group's slots
@@ -1132,7 +1130,7 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
                                    (abase[j1 + 1] - abase[j0]) * L * sizeof(SkEntry) <= GROUP_BYTES))
                     j1++;
                 if (nn - j1 < GROUP_FEATS / 2) j1 = nn;  // no short last group
-                groups.push_back({j0, j1, {}, {}, {}});
+                groups.push_back({j0, j1});
                 na = std::max(na, abase[j1] - abase[j0]);
                 nb = std::max(nb, bbase[j1] - bbase[j0]);
                 nt = std::max(nt, tbase[j1] - tbase[j0]);
@@ -1162,11 +1160,28 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
                     *c = cB + b + k;
                 }
             };
+            const uint32_t cut_lds = 4 * (uint32_t)L + 4 * max_bin;
+            sk_check(allow_lds(sk_cuts_kernel), "LDS attribute");
+            sk_check(allow_lds(sk_merge_kernel), "LDS attribute");
+            // Room for every group's tables: at most a pruning merge a batch, and fewer
+            // final merges than slots for them.
+            uint8_t *tab = s->alloc<uint8_t>(sizeof(SkSortTask) * abase[nn] +
+                                                 sizeof(SkMergeTask) * (abase[nn] + tbase[nn]) +
+                                                 sizeof(SkCutTask) * (uint64_t)nn,
+                                             "sketch task tables");
             std::vector<SkSortTask> sorts;
-            sorts.reserve(abase[nn]);
             std::vector<SkMergeTask> merges;
-            merges.reserve(abase[nn]);
-            for (Group &g : groups) {
+            std::vector<uint64_t> level_end;  // merges of levels 0..l end at level_end[l]
+            std::vector<std::vector<SkMergeTask>> finals;
+            std::vector<SkCutTask> cut_tasks;
+            std::vector<uint8_t> host;
+            // A group's tables are built and sent while the groups before it run.
+            for (const Group &g : groups) {
+                sorts.clear();
+                merges.clear();
+                level_end.clear();
+                finals.clear();
+                cut_tasks.clear();
                 for (uint32_t j = g.j0; j < g.j1; j++) {
                     const uint64_t a = abase[j] - abase[g.j0];
                     for (uint64_t k = 0; k < m[j]; k++) {
@@ -1175,6 +1190,7 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
                                                    A + (a + k) * L, cA + a + k, (uint32_t)len, 0});
                     }
                 }
+                if (sorts.empty()) continue;
                 for (uint32_t l = 0;; l++) {
                     bool any = false;
                     for (uint32_t j = g.j0; j < g.j1; j++) {
@@ -1197,19 +1213,14 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
                         }
                     }
                     if (!any) break;
-                    g.level_end.push_back(merges.size());
+                    level_end.push_back(merges.size());
                 }
-            }
-            // collapse: the levels still held (the set bits of m), lowest first.
-            std::vector<SkCutTask> cut_tasks;
-            for (Group &g : groups) {
-                std::vector<std::vector<SkMergeTask>> &finals = g.finals;
+                // collapse: the levels still held (the set bits of m), lowest first.
                 for (uint32_t j = g.j0; j < g.j1; j++) {
                     if (!m[j]) continue;
                     const SkEntry *cur = nullptr;
                     uint32_t *cur_n = nullptr;
                     uint32_t step = 0;
-                    uint64_t acc = 0;  // entries the merged result may hold, in limits
                     for (uint32_t l = 0; (m[j] >> l) != 0; l++) {
                         if (!((m[j] >> l) & 1)) continue;
                         const SkEntry *e;
@@ -1218,10 +1229,8 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
                         if (!cur) {
                             cur = e;
                             cur_n = cnt;
-                            acc = 1;
                             continue;
                         }
-                        acc++;
                         if (finals.size() <= step) finals.emplace_back();
                         SkMergeTask t{};
                         t.a = cur;
@@ -1237,72 +1246,44 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
                         cur_n = t.nd;
                         step++;
                     }
-                    (void)acc;
                     cut_tasks.push_back(SkCutTask{cur, cur_n, P + (uint64_t)j * L,
                                                   d_cuts + (uint64_t)j * n_cuts, d_ncut + j, {0, 0}});
                 }
-            }
-            // One upload of every table.
-            uint64_t n_final = 0;
-            for (const Group &g : groups)
-                for (const auto &f : g.finals) n_final += f.size();
-            const uint64_t bytes = sizeof(SkSortTask) * sorts.size() +
-                                   sizeof(SkMergeTask) * (merges.size() + n_final) +
-                                   sizeof(SkCutTask) * cut_tasks.size();
-            uint8_t *tab = s->alloc<uint8_t>(bytes, "sketch task tables");
-            std::vector<uint8_t> host(bytes);
-            uint64_t pos = 0;
-            auto put = [&](const void *p, uint64_t nb) {
-                if (nb) std::memcpy(host.data() + pos, p, nb);
-                pos += nb;
-            };
-            const uint64_t o_sort = pos;
-            put(sorts.data(), sizeof(SkSortTask) * sorts.size());
-            const uint64_t o_merge = pos;
-            put(merges.data(), sizeof(SkMergeTask) * merges.size());
-            for (Group &g : groups)
-                for (const auto &f : g.finals) {
-                    g.o_final.push_back(pos);
-                    put(f.data(), sizeof(SkMergeTask) * f.size());
-                }
-            const uint64_t o_cut = pos;
-            put(cut_tasks.data(), sizeof(SkCutTask) * cut_tasks.size());
-            sk_check(hipMemcpy(tab, host.data(), bytes, hipMemcpyHostToDevice), "task upload");
+                host.clear();
+                auto put = [&](const auto &v) {
+                    const uint64_t at = host.size(), nb = sizeof(v[0]) * v.size();
+                    host.resize(at + nb);
+                    if (nb) std::memcpy(host.data() + at, v.data(), nb);
+                    return tab + at;
+                };
+                const auto *d_sorts = reinterpret_cast<const SkSortTask *>(put(sorts));
+                const auto *d_merges = reinterpret_cast<const SkMergeTask *>(put(merges));
+                std::vector<const SkMergeTask *> d_finals;
+                for (const auto &f : finals)
+                    d_finals.push_back(reinterpret_cast<const SkMergeTask *>(put(f)));
+                const auto *d_cut_tasks = reinterpret_cast<const SkCutTask *>(put(cut_tasks));
+                sk_check(hipMemcpy(tab, host.data(), host.size(), hipMemcpyHostToDevice),
+                         "task upload");
+                tab += host.size();
 
-            // ---- launches ----
-            const uint32_t cut_lds = 4 * (uint32_t)L + 4 * max_bin;
-            sk_check(allow_lds(sk_cuts_kernel), "LDS attribute");
-            sk_check(allow_lds(sk_merge_kernel), "LDS attribute");
-            // Stream order: a group's cuts are taken before the next one's batches
-            // overwrite its summaries.
-            uint64_t first = 0, cut = 0;
-            for (const Group &g : groups) {
-                const uint64_t n_sort = abase[g.j1] - abase[g.j0];
-                if (!n_sort) continue;
-                launch_sort(reinterpret_cast<const SkSortTask *>(tab + o_sort) + abase[g.j0],
-                            (uint32_t)n_sort, (uint32_t)L, s->stream);
-                for (uint64_t e : g.level_end) {
+                // Stream order: a group's cuts are taken before the next one's batches
+                // overwrite its summaries.
+                launch_sort(d_sorts, (uint32_t)sorts.size(), (uint32_t)L, s->stream);
+                uint64_t first = 0;
+                for (uint64_t e : level_end) {
                     hipLaunchKernelGGL(sk_merge_kernel, dim3((uint32_t)(e - first)), dim3(SK_TPB),
-                                       2 * L, s->stream,
-                                       reinterpret_cast<const SkMergeTask *>(tab + o_merge) + first,
-                                       (uint32_t)L, 1u);
+                                       2 * L, s->stream, d_merges + first, (uint32_t)L, 1u);
                     sk_check(hipGetLastError(), "sketch merges");
                     first = e;
                 }
-                for (size_t t = 0; t < g.finals.size(); t++) {
-                    hipLaunchKernelGGL(sk_merge_kernel, dim3((uint32_t)g.finals[t].size()),
-                                       dim3(SK_TPB), 0, s->stream,
-                                       reinterpret_cast<const SkMergeTask *>(tab + g.o_final[t]),
-                                       (uint32_t)L, 0u);
+                for (size_t t = 0; t < finals.size(); t++) {
+                    hipLaunchKernelGGL(sk_merge_kernel, dim3((uint32_t)finals[t].size()),
+                                       dim3(SK_TPB), 0, s->stream, d_finals[t], (uint32_t)L, 0u);
                     sk_check(hipGetLastError(), "sketch final merges");
                 }
-                uint32_t n_cut = 0;
-                for (uint32_t j = g.j0; j < g.j1; j++) n_cut += m[j] ? 1u : 0u;
-                hipLaunchKernelGGL(sk_cuts_kernel, dim3(n_cut), dim3(SK_TPB), cut_lds, s->stream,
-                                   reinterpret_cast<const SkCutTask *>(tab + o_cut) + cut,
-                                   (uint32_t)L, max_bin);
+                hipLaunchKernelGGL(sk_cuts_kernel, dim3((uint32_t)cut_tasks.size()), dim3(SK_TPB),
+                                   cut_lds, s->stream, d_cut_tasks, (uint32_t)L, max_bin);
                 sk_check(hipGetLastError(), "sketch cuts");
-                cut += n_cut;
             }
             cuts_dev.resize((uint64_t)nn * n_cuts);
             sk_check(hipMemcpyAsync(n_out.data(), d_ncut, 4ull * nn, hipMemcpyDeviceToHost,
