@@ -299,11 +299,7 @@ struct fbh_ctx {
     bool rows_identity = false;
     double *red_f64 = nullptr;
     int64_t *red_i64 = nullptr;
-    // Blocks of the bounds and quantisation passes, whose results reduce_max_kernel and
-    // grow_prep_kernel go through on one workgroup: a row a thread, and rows in turn
-    // from 8192 blocks on. With 8192 at any size the four kernels took 40 us a tree of
-    // 5000 rows, now 16.
-    uint32_t n_red_blocks = 8192;
+    uint32_t n_red_blocks = 0;  // reduction_blocks(n_rows)
 
     // launch tables (device) and their pinned staging
     TileDev *d_tiles = nullptr;
@@ -917,8 +913,9 @@ void fixed_allocations(fbh_ctx &c, A &&a) {
     c.flags = static_cast<uint8_t *>(a(n, "partition flags"));
     c.hist = static_cast<int64_t *>(a(16 * (uint64_t)c.n_slots * c.width_max, "histogram slots"));
     c.d_scales = static_cast<ScalesDev *>(a(sizeof(ScalesDev), "quantizer scales"));
-    c.red_f64 = static_cast<double *>(a(8 * (2 * (uint64_t)c.n_red_blocks + 2), "reduction scratch"));
-    c.red_i64 = static_cast<int64_t *>(a(8 * (2 * (uint64_t)c.n_red_blocks + 2), "reduction scratch"));
+    const uint64_t red_bytes = 8 * reduction_words(c.n_red_blocks);
+    c.red_f64 = static_cast<double *>(a(red_bytes, "reduction scratch"));
+    c.red_i64 = static_cast<int64_t *>(a(red_bytes, "reduction scratch"));
     // The per-tree tables (tiles, tile features, split features) share one
     // buffer so that a tree's plan goes to the device in one copy.
     c.off_tilefeats = al256(sizeof(TileDev) * c.tiles.size());
@@ -1105,7 +1102,7 @@ fbh_config configure(fbh_ctx &c, uint64_t n_rows, const fbh_shape *shape, const 
         throw InputError("training data has " + std::to_string(n_rows) +
                          " rows, above the supported limit 4294967295");
     c.n_rows = n_rows;
-    c.n_red_blocks = (uint32_t)std::min<uint64_t>((n_rows + 255) / 256, 8192);
+    c.n_red_blocks = reduction_blocks(n_rows);
     c.n_features = shape->n_features;
     c.width.assign(shape->width, shape->width + shape->n_features);
     c.n_bins.assign(shape->n_bins, shape->n_bins + shape->n_features);

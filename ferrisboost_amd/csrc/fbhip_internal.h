@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fbhip_host.h"
+
 namespace fbh {
 
 // Memory and streams that jobs take and give back (fbhip_keep.hip). Calls act on

@@ -2748,7 +2748,6 @@ hipError_t launch_quantile_set(float2 *slot, float scale, float alpha, hipStream
 // threads sums its grid-stride rows in double, a fixed tree sums each
 // block, and one workgroup sums the block partials the same way, so every
 // run gives the same scale (not the host's serial sum).
-constexpr uint32_t QUANTILE_BLOCKS = 256;
 
 __global__ __launch_bounds__(256) void quantile_partials_kernel(const float *margin,
                                                                 const float *y, const float *w,

@@ -130,6 +130,21 @@ def test_full_size_first_rounds_equal_oracle(fb, oracle, alpha):
                           om.train_margins(y.size).view(np.uint32))
 
 
+@pytest.mark.parametrize("rows", [7, 300, 5_000, 65_024, 65_025])
+def test_fast_mode_with_few_rows(fb, rows):
+    """The device scale sums 256 blocks at any row count, also where a job needs
+    fewer for its gradients. Trees of one leaf (no split near a tie) are as close to
+    the exact mode's as the models of 50,000 rows are."""
+    x, y, _ = _data(rows, seed=3)
+    p = {"objective": "reg:quantileerror", "quantile_alpha": [0.2, 0.8], "gpu_math": "fast"}
+    for depth in (0, 3):
+        a, b = (fb.train(dict(p, max_depth=depth), x, y, num_boost_round=3) for _ in range(2))
+        assert a.to_json() == b.to_json()
+    fast, exact = (fb.train(dict(p, max_depth=0, gpu_math=m), x, y, num_boost_round=3)
+                   .predict(x, output_margin=True) for m in ("fast", "exact"))
+    assert np.abs(fast - exact).max() < 1e-3 * max(1.0, np.abs(exact).max())
+
+
 def test_fast_mode_is_deterministic_and_close(fb):
     x, y, _ = _data(50_000, seed=3)
     p = {"objective": "reg:quantileerror", "quantile_alpha": [0.2, 0.8], "max_depth": 6,
