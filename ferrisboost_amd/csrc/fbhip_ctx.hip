@@ -711,11 +711,9 @@ int64_t *fbh_ctx::partial_buffer(uint64_t bytes) {
     // Outside the memory plan: only within the budget's remaining room.
     if (bytes > partial_bytes && device_bytes - partial_bytes + bytes + 256 > plan.budget)
         return nullptr;
-    if (bytes > partial_bytes) {
-        release_alloc(partials);
-        partials = alloc<int64_t>(bytes / 8 + 1, "partial histograms");
-        partial_bytes = bytes;
-    }
+    regrow(
+        partials, partial_bytes, bytes, [&](int64_t *p) { release_alloc(p); },
+        [&](uint64_t b) { return alloc<int64_t>(b / 8 + 1, "partial histograms"); });
     return partials;
 }
 
@@ -1388,9 +1386,9 @@ static bool pack_rows(fbh_ctx &c, const std::vector<RowLayout> &layouts) {
     const uint64_t bytes = at + sizeof(PackCellDev) * cells.size();
     if (c.pack_tab_bytes < bytes) {
         if (c.device_bytes + bytes + 256 > c.plan.budget) return false;
-        c.release_alloc(c.pack_tab);
-        c.pack_tab = c.alloc<uint8_t>(bytes, "row packing table");
-        c.pack_tab_bytes = bytes;
+        regrow(
+            c.pack_tab, c.pack_tab_bytes, bytes, [&](uint8_t *p) { c.release_alloc(p); },
+            [&](uint64_t b) { return c.alloc<uint8_t>(b, "row packing table"); });
     }
     std::vector<uint8_t> tab(bytes);
     std::memcpy(tab.data(), rows.data(), sizeof(PackRowsDev) * rows.size());

@@ -25,4 +25,18 @@ inline uint64_t reduction_words(uint32_t n_red_blocks) {
     return std::max<uint64_t>(2ull * n_red_blocks + 2, 2ull * QUANTILE_BLOCKS);
 }
 
+// Replaces a kept buffer of `bytes` by one of at least `want` where it is smaller. The
+// old one is forgotten before the new one is asked for: when `take` throws, nothing
+// points to memory that has been given back, and a later call asks again.
+template <class T, class Release, class Take>
+void regrow(T *&p, uint64_t &bytes, uint64_t want, Release &&release, Take &&take) {
+    if (bytes >= want) return;
+    T *old = p;
+    p = nullptr;
+    bytes = 0;
+    release(old);
+    p = take(want);
+    bytes = want;
+}
+
 }  // namespace fbh

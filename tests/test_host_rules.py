@@ -39,3 +39,29 @@ def test_reduction_scratch_holds_every_pass(tmp_path):
         CHECK(reduction_words(b) >= 2ull * b + 2);
         CHECK(reduction_words(b) >= 2ull * QUANTILE_BLOCKS);
     }""")
+
+
+def test_a_failed_regrow_leaves_no_pointer(tmp_path):
+    """A kept table whose larger replacement cannot be allocated: the next request,
+    also one that the old size would have served, allocates again."""
+    run_cpp(tmp_path, """
+    std::vector<int *> freed;
+    int blocks[3];
+    int *p = &blocks[0];
+    uint64_t bytes = 64, taken = 0;
+    const auto release = [&](int *q) { freed.push_back(q); };
+    bool failed = false;
+    try {
+        regrow(p, bytes, 128, release, [&](uint64_t) -> int * { throw 1; });
+    } catch (int) {
+        failed = true;
+    }
+    CHECK(failed && p == nullptr && bytes == 0);
+    CHECK(freed.size() == 1 && freed[0] == &blocks[0]);
+    const auto take = [&](uint64_t b) { taken = b; return &blocks[1]; };
+    regrow(p, bytes, 64, release, take);
+    CHECK(p == &blocks[1] && bytes == 64 && taken == 64);
+    taken = 0;
+    regrow(p, bytes, 32, release, take);
+    CHECK(p == &blocks[1] && bytes == 64 && taken == 0);
+    CHECK(freed.size() == 2 && freed[1] == nullptr);""")
