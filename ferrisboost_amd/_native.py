@@ -428,6 +428,7 @@ def train_lib() -> C.CDLL:
 
 # fbt_predict outputs (include/fbtrain.h).
 OUT_MARGIN, OUT_VALUE, OUT_LEAF, OUT_CONTRIBS, OUT_APPROX, OUT_INTERACTIONS = range(6)
+ORDER_ENGINE, ORDER_SUMS = 0x100, 0x200
 
 
 def ptr(a):

@@ -14,9 +14,11 @@
 //     pair;
 //   * the cover-weighted mean of every node in f32 (fill_node_means,
 //     src/model/explain.rs:409-422) for Saabas.
-// Every kernel gives one thread one row and walks the trees in model order,
-// with the host engine's float32 operations in the host engine's order, so
-// results equal the CPU's bit for bit.
+// The kernels here give one thread one row and walk the trees in model order,
+// with the host engine's float32 operations in the host engine's order, so their
+// results equal the CPU's bit for bit. They take what fbhip_shap_paths.hip (TreeSHAP
+// of trees of at most 8 levels by closed sums, in another order) and fbhip_predict.hip
+// (the same additions as here) do not, and TreeSHAP under fbh_shap_set_host_order.
 
 #include "fbhip_internal.h"
 #include "fb_expf.h"

@@ -452,17 +452,12 @@ void sort_row_ascending(float *row, uint32_t k) {
     }
 }
 
-// Explanations of fewer rows of a multi-output model keep the host engine's
-// operation order: small samples are compared with its per-class values bit for
-// bit. Larger ones take the backend's default.
-constexpr uint64_t HOST_ORDER_ROWS = 512;
-
 // A multiclass model's outputs: each class scored or explained by its own
 // trees with its own intercept (Model::class_view, src/model/tree.rs:
 // 395-425), the per-class results laid out [row][class][...].
 void predict_multiclass(const fbt_model &mm, const float *x, uint64_t n_rows, uint32_t nf,
-                        uint32_t output, uint32_t begin, uint32_t end, const float *base_margin,
-                        int device, float *out) {
+                        uint32_t output, bool engine_order, uint32_t begin, uint32_t end,
+                        const float *base_margin, int device, float *out) {
     const fbt::Model &m = mm.m;
     const uint32_t K = m.n_outputs();
     if (output == FBT_OUT_LEAF) {
@@ -491,7 +486,7 @@ void predict_multiclass(const fbt_model &mm, const float *x, uint64_t n_rows, ui
             }
         } else {
             DeviceModel sm(mm, begin, end, k, device);
-            int rc = fbh_shap_set_host_order(sm.get(), !scores && n_rows < HOST_ORDER_ROWS);
+            int rc = fbh_shap_set_host_order(sm.get(), engine_order);
             if (rc) backend_fail(rc);
             if (scores) rc = fbh_predict(sm.get(), x, n_rows, bm, FBH_PREDICT_MARGIN, col.data());
             else if (output == FBT_OUT_CONTRIBS) rc = fbh_shap_contribs(sm.get(), x, n_rows, bm, col.data());
@@ -525,8 +520,8 @@ void predict_multiclass(const fbt_model &mm, const float *x, uint64_t n_rows, ui
 
 // A single-output model's outputs.
 void predict_single(const fbt_model &mm, const float *x, uint64_t n_rows, uint32_t nf,
-                    uint32_t output, uint32_t begin, uint32_t end, const float *base_margin,
-                    int device, float *out) {
+                    uint32_t output, bool engine_order, uint32_t begin, uint32_t end,
+                    const float *base_margin, int device, float *out) {
     const fbt::Model &m = mm.m;
     const bool logistic = m.objective == 1;
     if (device < 0) {
@@ -543,7 +538,8 @@ void predict_single(const fbt_model &mm, const float *x, uint64_t n_rows, uint32
         return;
     }
     DeviceModel sm(mm, begin, end, DeviceModels::ALL, device);
-    int rc = FBH_OK;
+    int rc = fbh_shap_set_host_order(sm.get(), engine_order);
+    if (rc) backend_fail(rc);
     switch (output) {
         case FBT_OUT_MARGIN:
             rc = fbh_predict(sm.get(), x, n_rows, base_margin, FBH_PREDICT_MARGIN, out);
@@ -588,7 +584,14 @@ int fbt_predict(const fbt_model *mm, const float *x, uint64_t n_rows, uint32_t n
         if (n_features != m.n_features)
             throw fbt::InputError("expected " + std::to_string(m.n_features) + " features, got " +
                                   std::to_string(n_features));
-        if (output > FBT_OUT_INTERACTIONS) throw fbt::InputError("unknown prediction output");
+        const uint32_t order = output & (FBT_ORDER_ENGINE | FBT_ORDER_SUMS);
+        output &= ~order;
+        if (output > FBT_OUT_INTERACTIONS || order == (FBT_ORDER_ENGINE | FBT_ORDER_SUMS) ||
+            (order && output != FBT_OUT_CONTRIBS && output != FBT_OUT_INTERACTIONS))
+            throw fbt::InputError("unknown prediction output");
+        // One order for a model whatever the call's size, so that a row's values do not
+        // depend on the batch it is explained in.
+        const bool engine = order ? order == FBT_ORDER_ENGINE : m.n_outputs() > 1;
         if (tree_begin > tree_end || tree_end > m.trees.size())
             throw fbt::InputError("tree range [" + std::to_string(tree_begin) + ", " +
                                   std::to_string(tree_end) + ") is outside the model's " +
@@ -596,10 +599,10 @@ int fbt_predict(const fbt_model *mm, const float *x, uint64_t n_rows, uint32_t n
         ReservedCheck reserved(x, n_rows * (uint64_t)n_features);
         try {
             if (m.n_outputs() > 1)
-                predict_multiclass(*mm, x, n_rows, n_features, output, tree_begin, tree_end,
-                                   base_margin, device, out);
+                predict_multiclass(*mm, x, n_rows, n_features, output, engine, tree_begin,
+                                   tree_end, base_margin, device, out);
             else
-                predict_single(*mm, x, n_rows, n_features, output, tree_begin, tree_end,
+                predict_single(*mm, x, n_rows, n_features, output, engine, tree_begin, tree_end,
                                base_margin, device, out);
         } catch (...) {
             reserved.check();  // a reserved value is the error to report

@@ -241,6 +241,12 @@ enum {
      * intercept (Model::class_view, src/model/tree.rs:395-425): contributions
      * [n_rows][K][n_features + 1], interactions [n_rows][K][...]^2. */
 };
+/* Or-ed to FBT_OUT_CONTRIBS or FBT_OUT_INTERACTIONS, at most one: TreeSHAP with
+ * the engine's float operations in its order (equal to the CPU engine's bit for
+ * bit), or by closed sums (fbh_shap_set_host_order: faster, within 1e-5 of the
+ * engine's and closer to exact arithmetic). With neither, a single-output model
+ * takes the sums and a multi-output one the engine's order, at any row count. */
+enum { FBT_ORDER_ENGINE = 0x100, FBT_ORDER_SUMS = 0x200 };
 /* Model.predict (python/ferrisboost/_core.pyi:94-197, src/python/mod.rs:
  * 2667-2800) over the trees [tree_begin, tree_end) (n_trees and
  * iteration_range select them: a prefix, or the slice of
