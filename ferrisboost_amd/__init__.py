@@ -28,7 +28,7 @@ import numpy as np
 from . import _native as N
 from . import frame_rows
 
-__all__ = ["train", "sketch", "Cuts", "Model", "device_available", "__version__"]
+__all__ = ["train", "sketch", "Cuts", "Model", "device_available", "release_cached", "__version__"]
 __version__ = "0.1.0"
 
 # Canonical name -> default, as python/ferrisboost/__init__.py:_DEFAULTS.
@@ -124,6 +124,14 @@ def _parse_device(value) -> int:
                 '(use device="cuda" or "cuda:N")'
             )
     raise ValueError(f'device must be "cuda" or "cuda:N", got {value!r}')
+
+
+def release_cached(device=None) -> None:
+    """Gives back the device memory, page-locked memory and streams that finished
+    training jobs and models between calls have left for the next ones (at most a
+    sixteenth of the device's memory, and 4 GiB of models). Nothing in use is
+    touched; later calls ask for theirs again."""
+    N.check_hip(N.hip().fbh_release_cached(_parse_device(device)))
 
 
 def _normalize(params: Mapping[str, Any], num_boost_round: int) -> dict[str, Any]:

@@ -236,7 +236,8 @@ HIP_SYMBOLS = [
     "fbh_hist_timing", "fbh_set_timing", "fbh_build_histogram", "fbh_partition_rows",
     "fbh_shap_model_create", "fbh_shap_model_destroy", "fbh_shap_contribs",
     "fbh_shap_contribs_device", "fbh_shap_last_ms", "fbh_shap_interactions",
-    "fbh_shap_set_host_order", "fbh_release_cached",
+    "fbh_shap_set_host_order", "fbh_release_cached", "fbh_shap_model_park",
+    "fbh_shap_model_unpark", "fbh_shap_models_drop",
     "fbh_saabas_contribs", "fbh_predict", "fbh_predict_device", "fbh_shap_contribs_noalloc",
 ]
 TRAIN_SYMBOLS = [
@@ -347,6 +348,10 @@ def hip() -> C.CDLL:
         L.fbh_shap_model_destroy.argtypes = [P]
         L.fbh_shap_set_host_order.argtypes = [P, C.c_int]
         L.fbh_release_cached.argtypes = [C.c_int]
+        L.fbh_shap_model_park.argtypes = [P, C.c_uint64, C.c_uint64, C.c_uint32]
+        L.fbh_shap_model_unpark.argtypes = [C.c_int, C.c_uint64, C.c_uint64, C.c_uint32,
+                                            C.POINTER(P)]
+        L.fbh_shap_models_drop.argtypes = [C.c_uint64]
         L.fbh_sketch_rows.argtypes = [P, C.POINTER(P)]
         L.fbh_bin_rows.argtypes = [P, P, C.c_uint64, C.c_uint64]
         L.fbh_shap_contribs.argtypes = [P, P, C.c_uint64, P, P]

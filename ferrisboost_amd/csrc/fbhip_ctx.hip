@@ -523,7 +523,7 @@ struct fbh_ctx {
         if (leaves_done) (void)hipEventDestroy(leaves_done);
         leaves_done = nullptr;
         for (hipStream_t *s : {&copy_stream, &up_stream, &stream}) {
-            keep_stream_back(device, *s);
+            (void)keep_stream_back(device, *s);
             *s = nullptr;
         }
     }

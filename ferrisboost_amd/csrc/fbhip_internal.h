@@ -17,8 +17,10 @@ hipError_t keep_alloc(KeepKind kind, void **p, uint64_t bytes);
 void keep_free(KeepKind kind, void *p, bool keep = true) noexcept;
 bool keep_release(int device) noexcept;     // frees what is kept; whether there was any
 uint64_t keep_bytes(int device) noexcept;   // device memory kept
+bool drop_parked(int device) noexcept;      // destroys parked models (fbhip_shap.hip);
+uint64_t parked_bytes(int device) noexcept; // whether there were any; their memory
 hipError_t keep_stream(hipStream_t *s);     // a non-blocking stream
-void keep_stream_back(int device, hipStream_t s) noexcept;  // waits for it
+hipError_t keep_stream_back(int device, hipStream_t s) noexcept;  // waits for it
 
 constexpr int HIST_TPB = 256;      // threads of one histogram workgroup
 constexpr int SPLIT_TPB = 256;     // threads of one split-scan workgroup

@@ -13,7 +13,7 @@
 // Blocks serve requests of their own size alone, so nobody holds more memory than
 // was asked for. A device keeps at most a sixteenth of its memory, the oldest
 // blocks beyond that go; a failed allocation, an object with a memory budget and
-// fbh_release_cached give everything back. Who gives a block or a stream back has
+// fbh_release_cached give everything back, parked models (fbh_shap_model_park) first. Who gives a block or a stream back has
 // waited for all work on it, so any thread and stream can take it next. Contents
 // are those of the last use, as of any block that hipMalloc cuts from a page in use.
 #include <hip/hip_runtime.h>
@@ -172,7 +172,8 @@ void keep_free(KeepKind kind, void *p, bool keep) noexcept {
 }
 
 bool keep_release(int device) noexcept {
-    if (device < 0 || device >= MAX_KEEP_DEVICES) return false;
+    const bool models = drop_parked(device);  // (their memory is kept, and goes below)
+    if (device < 0 || device >= MAX_KEEP_DEVICES) return models;
     Kept &k = kept();
     std::vector<Block> in;
     std::vector<hipStream_t> streams;
@@ -184,14 +185,15 @@ bool keep_release(int device) noexcept {
     }
     for (const Block &b : in) give_back(b);
     for (hipStream_t s : streams) (void)hipStreamDestroy(s);
-    return !in.empty();
+    return models || !in.empty();
 }
 
 uint64_t keep_bytes(int device) noexcept {
-    if (device < 0 || device >= MAX_KEEP_DEVICES) return 0;
+    const uint64_t models = parked_bytes(device);
+    if (device < 0 || device >= MAX_KEEP_DEVICES) return models;
     Kept &k = kept();
     std::lock_guard<std::mutex> g(k.mu);
-    return k.bytes[device];
+    return models + k.bytes[device];
 }
 
 hipError_t keep_stream(hipStream_t *s) {
@@ -210,21 +212,23 @@ hipError_t keep_stream(hipStream_t *s) {
     return hipStreamCreateWithFlags(s, hipStreamNonBlocking);
 }
 
-void keep_stream_back(int device, hipStream_t s) noexcept {
-    if (!s) return;
+hipError_t keep_stream_back(int device, hipStream_t s) noexcept {
+    if (!s) return hipSuccess;
     // Waits for it; a stream that reports an error is not handed on.
-    if (hipStreamSynchronize(s) == hipSuccess && device >= 0 && device < MAX_KEEP_DEVICES) {
+    const hipError_t e = hipStreamSynchronize(s);
+    if (e == hipSuccess && device >= 0 && device < MAX_KEEP_DEVICES) {
         Kept &k = kept();
         std::lock_guard<std::mutex> g(k.mu);
         try {
             if (k.streams[device].size() < STREAMS_MOST) {
                 k.streams[device].push_back(s);
-                return;
+                return e;
             }
         } catch (...) {
         }
     }
     (void)hipStreamDestroy(s);
+    return e;
 }
 
 }  // namespace fbh

@@ -778,19 +778,37 @@ struct fbh_shap_model {
     // between calls; host_mu is held by the call that uses them.
     std::mutex host_mu;
     void *staging = nullptr, *pinned = nullptr;
-    uint64_t staging_bytes = 0;
+    uint64_t staging_bytes = 0, array_bytes = 0;
+    static constexpr uint64_t SMALL_WORK = 1 << 20;
 
     ~fbh_shap_model() {
         if (device >= 0) (void)hipSetDevice(device);
-        if (stream) (void)hipStreamSynchronize(stream);
+        (void)rest(true);
         for (void *p : allocs) keep_free(KeepKind::device, p);
-        keep_free(KeepKind::device, work);
-        keep_free(KeepKind::device, staging);
-        keep_free(KeepKind::host, pinned);
         if (e0) (void)hipEventDestroy(e0);
         if (e1) (void)hipEventDestroy(e1);
-        keep_stream_back(device, stream);
     }
+    // Waits for the stream and gives back what a call needs beside the arrays, which
+    // the next one asks for again; `all` but what a few rows need (a block of
+    // page-locked memory, a small workspace), which is not worth that.
+    hipError_t rest(bool all) noexcept {
+        const hipError_t e = keep_stream_back(device, stream);
+        stream = nullptr;
+        if (all || work_bytes > SMALL_WORK) {
+            keep_free(KeepKind::device, work);
+            work = nullptr;
+            work_bytes = 0;
+        }
+        keep_free(KeepKind::device, staging);
+        staging = nullptr;
+        staging_bytes = 0;
+        if (all) {
+            keep_free(KeepKind::host, pinned);
+            pinned = nullptr;
+        }
+        return e;
+    }
+    uint64_t held_bytes() const { return array_bytes + work_bytes + staging_bytes; }
     // The arrays added so far, laid out in one allocation and sent in one copy.
     struct Arrays {
         std::vector<unsigned char> bytes;
@@ -807,6 +825,7 @@ struct fbh_shap_model {
         void *p = nullptr;
         chk(keep_alloc(KeepKind::device, &p, a.bytes.size()), "model arrays");
         allocs.push_back(p);
+        array_bytes += a.bytes.size();
         chk(hipMemcpy(p, a.bytes.data(), a.bytes.size(), hipMemcpyHostToDevice), "model arrays");
         for (const auto &f : a.place) f(static_cast<unsigned char *>(p));
     }
@@ -1061,11 +1080,23 @@ bool takes_paths(const fbh_shap_model *m, bool inter) {
 // trees of depth 8 at once, which is nine times what fills the device.
 constexpr uint64_t PATHS_WORK_BYTES = 512ull << 20;
 
+// Blocks that a call asks for and gives back serve requests of their own size alone
+// (fbhip_keep.hip): powers of two, from 64 MiB multiples of it, so that calls of
+// other row counts find them.
+uint64_t block_size(uint64_t bytes) {
+    constexpr uint64_t STEP = 64ull << 20;
+    if (bytes > STEP) return (bytes + STEP - 1) / STEP * STEP;
+    uint64_t b = 64 << 10;
+    while (b < bytes) b *= 2;
+    return b;
+}
+
 // Grows the model's workspace to `want` bytes, or to as much as there is, not
 // below `least`; work_mu must be held. Work of earlier calls runs on the same
 // stream before this one's, so calls share the workspace.
 bool grow_work(fbh_shap_model *m, uint64_t want, uint64_t least) {
     if (m->work_bytes >= want) return true;
+    want = block_size(want);
     if (m->work) {
         chk(hipStreamSynchronize(m->stream), "workspace");
         keep_free(KeepKind::device, m->work);
@@ -1304,7 +1335,7 @@ void run_host_alloc(fbh_shap_model *m, Kind k, const float *rows, uint64_t n_row
     st.cap_rows = std::min<uint64_t>(n_rows, std::max<uint64_t>(1, (512ull << 20) / per_row));
     const uint64_t o_rows = round256(4 * st.cap_rows * nf);
     const uint64_t o_out = o_rows + round256(4 * st.cap_rows);
-    const uint64_t need = o_out + 4 * st.cap_rows * w + 4;
+    const uint64_t need = block_size(o_out + 4 * st.cap_rows * w + 4);
     // A call's own staging goes back once the stream is done with it.
     auto give_back = [m](void *p) {
         (void)hipStreamSynchronize(m->stream);
@@ -1353,9 +1384,136 @@ void *scratch_of(int device) {
     return g_scratch_ptr[device];
 }
 
+// Models that their owners leave here between calls, oldest first.
+struct Parked {
+    uint64_t owner, trees;
+    uint32_t output;
+    fbh_shap_model *m;
+    bool is(int device, uint64_t o, uint64_t t, uint32_t out) const {
+        return m->device == device && owner == o && trees == t && output == out;
+    }
+};
+struct Parking {
+    std::mutex mu;
+    std::vector<Parked> in;
+    // Most a device's parked models hold, and most of them (each with a page-locked
+    // block of PINNED_BYTES): arrays of 100 trees of depth 8 are 8 MiB, and a model of
+    // many classes or tree ranges parks one each.
+    static constexpr uint64_t BYTES_MOST = 4ull << 30;
+    static constexpr size_t MODELS_MOST = 256;
+};
+
+// Never destroyed, as the kept memory.
+Parking &parking() {
+    static Parking *p = new Parking;
+    return *p;
+}
+
+// Takes the models out that `leave` picks, and destroys them outside the lock with
+// the caller's device current afterwards.
+template <class F>
+bool drop_models(F &&leave) noexcept {
+    std::vector<Parked> out;
+    Parking &P = parking();
+    try {
+        std::lock_guard<std::mutex> g(P.mu);
+        out.reserve(P.in.size());
+        for (size_t i = 0; i < P.in.size();)
+            if (leave(P.in[i])) {
+                out.push_back(P.in[i]);
+                P.in.erase(P.in.begin() + (ptrdiff_t)i);
+            } else {
+                i++;
+            }
+    } catch (const std::bad_alloc &) {  // nothing was taken out
+    }
+    if (out.empty()) return false;
+    int dev = -1;
+    const bool known = hipGetDevice(&dev) == hipSuccess;
+    for (const Parked &p : out) delete p.m;
+    if (known) (void)hipSetDevice(dev);
+    return true;
+}
+
 }  // namespace
 
+namespace fbh {
+
+bool drop_parked(int device) noexcept {
+    return drop_models([&](const Parked &p) { return p.m->device == device; });
+}
+
+uint64_t parked_bytes(int device) noexcept {
+    Parking &P = parking();
+    std::lock_guard<std::mutex> g(P.mu);
+    uint64_t b = 0;
+    for (const Parked &p : P.in)
+        if (p.m->device == device) b += p.m->held_bytes();
+    return b;
+}
+
+}  // namespace fbh
+
 extern "C" {
+
+int fbh_shap_model_park(fbh_shap_model *m, uint64_t owner, uint64_t trees, uint32_t output) {
+    return shap_guard([&] {
+        if (!m) throw ShapError(FBH_INPUT_ERROR, "null argument");
+        std::unique_ptr<fbh_shap_model> mine(m);  // goes where it cannot stay
+        const int device = m->device;
+        chk(hipSetDevice(device), "hipSetDevice");
+        chk(m->rest(false), "park");
+        uint64_t bytes = 0;
+        size_t n = 0;
+        {
+            Parking &P = parking();
+            std::lock_guard<std::mutex> g(P.mu);
+            P.in.push_back({owner, trees, output, m});
+            mine.release();
+            for (const Parked &p : P.in)
+                if (p.m->device == device) {
+                    bytes += p.m->held_bytes();
+                    n++;
+                }
+        }
+        if (bytes <= Parking::BYTES_MOST && n <= Parking::MODELS_MOST) return;
+        (void)drop_models([&](const Parked &p) {  // the oldest, until the others may stay
+            if (p.m->device != device || (bytes <= Parking::BYTES_MOST && n <= Parking::MODELS_MOST))
+                return false;
+            bytes -= p.m->held_bytes();
+            n--;
+            return true;
+        });
+    });
+}
+
+int fbh_shap_model_unpark(int device, uint64_t owner, uint64_t trees, uint32_t output,
+                          fbh_shap_model **out) {
+    return shap_guard([&] {
+        if (!out) throw ShapError(FBH_INPUT_ERROR, "null argument");
+        *out = nullptr;
+        std::unique_ptr<fbh_shap_model> m;
+        {
+            Parking &P = parking();
+            std::lock_guard<std::mutex> g(P.mu);
+            for (size_t i = 0; i < P.in.size(); i++)
+                if (P.in[i].is(device, owner, trees, output)) {
+                    m.reset(P.in[i].m);
+                    P.in.erase(P.in.begin() + (ptrdiff_t)i);
+                    break;
+                }
+        }
+        if (!m) return;
+        chk(hipSetDevice(device), "hipSetDevice");
+        chk(keep_stream(&m->stream), "stream");
+        *out = m.release();
+    });
+}
+
+int fbh_shap_models_drop(uint64_t owner) {
+    (void)drop_models([&](const Parked &p) { return p.owner == owner; });
+    return FBH_OK;
+}
 
 int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_offsets,
                           const uint32_t *feat, const float *split_cond, const int32_t *left,

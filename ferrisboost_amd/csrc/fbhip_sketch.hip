@@ -911,8 +911,8 @@ struct fbh_sketch {
         pipe.release();
         for (void *p : allocs) keep_free(KeepKind::device, p, keep);
         if (arrived) (void)hipEventDestroy(arrived);
-        keep_stream_back(device, copy);
-        keep_stream_back(device, stream);
+        (void)keep_stream_back(device, copy);
+        (void)keep_stream_back(device, stream);
     }
 };
 

@@ -1,12 +1,12 @@
 // fbt_api.cpp -- C ABI of the round driver (include/fbtrain.h).
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <future>
 #include <limits>
 #include <memory>
-#include <mutex>
 #include <string>
 #include <thread>
 #include <utility>
@@ -27,52 +27,24 @@ namespace {
 
 using ShapModel = std::unique_ptr<fbh_shap_model, int (*)(fbh_shap_model *)>;
 
-// The device models of a model's trees that predictions and explanations have
-// used, kept for the next call: one for a tree range, output and device. A call
-// takes its entry out and puts it back, so that calls from several threads each
-// work on a device model of their own; the oldest beyond KEEP are dropped.
-class DeviceModels {
-public:
-    struct Key {
-        uint32_t begin, end, output;  // output of a multi-output model, or ALL
-        int device;
-        bool operator==(const Key &o) const {
-            return begin == o.begin && end == o.end && output == o.output && device == o.device;
-        }
-    };
-    static constexpr uint32_t ALL = 0xFFFFFFFFu;
+constexpr uint32_t ALL_OUTPUTS = 0xFFFFFFFFu;
 
-    ShapModel take(const Key &k) {
-        std::lock_guard<std::mutex> g(mu_);
-        for (size_t i = 0; i < kept_.size(); i++)
-            if (kept_[i].first == k) {
-                ShapModel m = std::move(kept_[i].second);
-                kept_.erase(kept_.begin() + (ptrdiff_t)i);
-                return m;
-            }
-        return ShapModel(nullptr, fbh_shap_model_destroy);
-    }
-    void put(const Key &k, ShapModel m) {
-        ShapModel old(nullptr, fbh_shap_model_destroy);  // destroyed outside the lock
-        std::lock_guard<std::mutex> g(mu_);
-        kept_.emplace_back(k, std::move(m));
-        if (kept_.size() > KEEP) {
-            old = std::move(kept_.front().second);
-            kept_.erase(kept_.begin());
-        }
-    }
-
-private:
-    static constexpr size_t KEEP = 8;
-    std::mutex mu_;
-    std::vector<std::pair<Key, ShapModel>> kept_;
-};
+// A name for a model's parked device models that no other model has had.
+uint64_t next_owner() {
+    static std::atomic<uint64_t> n{1};
+    return n++;
+}
 
 }  // namespace
 
 struct fbt_model {
     fbt::Model m;
-    mutable DeviceModels device;
+    const uint64_t owner = next_owner();
+
+    fbt_model() = default;
+    fbt_model(const fbt_model &) = delete;
+    fbt_model &operator=(const fbt_model &) = delete;
+    ~fbt_model() { (void)fbh_shap_models_drop(owner); }
 };
 
 namespace {
@@ -338,13 +310,18 @@ ShapModel explain_model(const fbt::Model &m, const std::vector<uint32_t> &ids, f
 }
 
 // A call's use of the device model of the trees [begin, end) (of output `output`
-// alone, or of all): the kept one, or a new one, kept afterwards.
+// alone, or of all): the one an earlier call has parked, or a new one, parked
+// afterwards. Calls from several threads each work on a device model of their own.
 class DeviceModel {
 public:
     DeviceModel(const fbt_model &mm, uint32_t begin, uint32_t end, uint32_t output, int device)
-        : owner_(mm.device), key_{begin, end, output, device}, m_(mm.device.take(key_)) {
+        : owner_(mm.owner), trees_((uint64_t)begin << 32 | end), output_(output),
+          m_(nullptr, fbh_shap_model_destroy) {
+        fbh_shap_model *parked = nullptr;
+        if (int rc = fbh_shap_model_unpark(device, owner_, trees_, output_, &parked)) backend_fail(rc);
+        m_.reset(parked);
         if (m_) return;
-        const bool all = output == DeviceModels::ALL;
+        const bool all = output == ALL_OUTPUTS;
         const uint32_t K = mm.m.n_outputs();
         std::vector<uint32_t> ids;
         for (uint32_t t = begin; t < end; t++)
@@ -352,18 +329,15 @@ public:
         m_ = explain_model(mm.m, ids, all ? mm.m.base_margin() : mm.m.class_margins[output], device);
     }
     ~DeviceModel() {
-        try {
-            owner_.put(key_, std::move(m_));
-        } catch (...) {  // out of memory: the device model goes
-        }
+        if (m_) (void)fbh_shap_model_park(m_.release(), owner_, trees_, output_);
     }
     DeviceModel(const DeviceModel &) = delete;
     DeviceModel &operator=(const DeviceModel &) = delete;
     fbh_shap_model *get() const { return m_.get(); }
 
 private:
-    DeviceModels &owner_;
-    DeviceModels::Key key_;
+    uint64_t owner_, trees_;
+    uint32_t output_;
     ShapModel m_;
 };
 
@@ -462,7 +436,7 @@ void predict_multiclass(const fbt_model &mm, const float *x, uint64_t n_rows, ui
     const uint32_t K = m.n_outputs();
     if (output == FBT_OUT_LEAF) {
         if (device < 0) throw fbt::InputError("explanations run on the device; pass a device index");
-        DeviceModel sm(mm, begin, end, DeviceModels::ALL, device);
+        DeviceModel sm(mm, begin, end, ALL_OUTPUTS, device);
         if (int rc = fbh_predict(sm.get(), x, n_rows, nullptr, FBH_PREDICT_LEAF, out)) backend_fail(rc);
         g_last_shap_ms = fbh_shap_last_ms(sm.get());
         return;
@@ -537,7 +511,7 @@ void predict_single(const fbt_model &mm, const float *x, uint64_t n_rows, uint32
         }
         return;
     }
-    DeviceModel sm(mm, begin, end, DeviceModels::ALL, device);
+    DeviceModel sm(mm, begin, end, ALL_OUTPUTS, device);
     int rc = fbh_shap_set_host_order(sm.get(), engine_order);
     if (rc) backend_fail(rc);
     switch (output) {

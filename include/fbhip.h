@@ -136,8 +136,9 @@ size_t fbh_last_error(char *buf, size_t len);
 int fbh_device_available(int device);
 /* Contexts, sketches and models without a memory budget leave their buffers and
  * streams to the next one: at most a sixteenth of the device's memory, given back
- * when an allocation needs it, when something is made with a budget, or here.
- * Nothing in use is touched. No reference counterpart. */
+ * when an allocation needs it, when something is made with a budget, or here, and
+ * parked models (fbh_shap_model_park) with it. Nothing in use is touched. No
+ * reference counterpart. */
 int fbh_release_cached(int device);
 
 /* ------------------------------------------------------------ lifecycle */
@@ -623,6 +624,19 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
                           uint32_t n_cat_words, uint32_t n_features, float bias,
                           fbh_shap_model **out);
 int fbh_shap_model_destroy(fbh_shap_model *m);
+/* For callers that make device models for single calls: leaves one with the library
+ * until the same owner takes it again under the same name (its tree range and
+ * output, or any numbers the owner chooses). The caller's handle ends, on an error
+ * too. Staging, stream and a workspace above 1 MiB go back at once; the rest stays,
+ * at most 4 GiB and 256 models of a device, the oldest go first; and all of a
+ * device's parked models go where fbh_release_cached gives back what is kept. No
+ * reference counterpart. */
+int fbh_shap_model_park(fbh_shap_model *m, uint64_t owner, uint64_t trees, uint32_t output);
+/* The parked model, the caller's own again; *out NULL when it is not there. */
+int fbh_shap_model_unpark(int device, uint64_t owner, uint64_t trees, uint32_t output,
+                          fbh_shap_model **out);
+/* Destroys the owner's parked models. */
+int fbh_shap_models_drop(uint64_t owner);
 /* Contributions and interactions of trees of at most 8 split levels are taken
  * by default from closed sums of the same quadrature (no divides; the values of
  * exact arithmetic to within float rounding, closer than the host engine's
