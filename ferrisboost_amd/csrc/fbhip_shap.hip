@@ -881,8 +881,8 @@ float node_means(const std::vector<int32_t> &left, const std::vector<int32_t> &r
 }
 
 // The split nodes of a tree in preorder as fbhip_shap_paths.hip walks them; false
-// where its arithmetic would leave the range of a float (covers or leaf values
-// near its limits) or a threshold is NaN.
+// where its arithmetic would leave the range of a float (a path's weights, or a leaf
+// value times its path's weights, near its limits) or a threshold is NaN.
 struct PathBuild {
     std::vector<PathNodeDev> nodes;
     std::vector<PathTestDev> tests;
@@ -937,7 +937,12 @@ private:
             a[s] = (float)hot;
             if (!(hot > -1.0 && hot < 1e30)) ok = false;
             const ShapNodeDev &c = n[child[s]];
-            if (!(c.flags & 1u)) continue;
+            if (!(c.flags & 1u)) {
+                // the factors above it grow to 1 / (the weights above it), whatever
+                // the leaves below
+                if (weight * w[s] < 1e-36) ok = false;
+                continue;
+            }
             p.meta |= s ? PATH_LEAF_R : PATH_LEAF_L;
             const double leaf = (double)c.leaf_value * weight * w[s];
             v[s] = (float)leaf;

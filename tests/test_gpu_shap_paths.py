@@ -103,3 +103,51 @@ def test_paths_match_the_host_order(lib, rows, n_trees, depth, nf, n_cat, full):
                 assert np.max(np.abs(got - want)) <= t, (name, np.max(np.abs(got - want)), t)
     finally:
         N.hip().fbh_shap_model_destroy(h)
+
+
+@pytest.mark.parametrize("share,fits", [(1e-3, True), (1e-5, True), (1e-6, False)])
+def test_weights_near_the_range_of_a_float(lib, share, fits):
+    """A path of eight splits on as many features that each pass `share` of the cover
+    on, to leaves of value 0. The factors above its last split grow to 1e21, 1e35 and
+    1e42; the last is beyond a float, and the model takes the engine's order, whose
+    values it then has. The others stay finite and add up."""
+    N = lib
+    D = 8
+    n = 2 * D + 1
+    a = {"feat": np.zeros(n, np.uint32), "cond": np.zeros(n, np.float32),
+         "left": np.full(n, -1, np.int32), "right": np.full(n, -1, np.int32),
+         "dl": np.zeros(n, np.uint8), "leaf": np.ones(n, np.uint8),
+         "val": np.full(n, 0.5, np.float32), "hess": np.zeros(n, np.float32)}
+    at, a["hess"][0] = 0, 1e10
+    for d in range(D):
+        a["feat"][at], a["leaf"][at], a["val"][at] = d, 0, 0
+        a["left"][at], a["right"][at] = 2 * d + 1, 2 * d + 2
+        a["hess"][2 * d + 1] = a["hess"][at] * np.float32(share)
+        a["hess"][2 * d + 2] = a["hess"][at]
+        at = 2 * d + 1
+    a["val"][2 * (D - 2) + 1:] = 0.0  # every leaf below the sixth split
+    offs = np.array([0, n], np.uint32)
+    h = C.c_void_p()
+    N.check_hip(N.hip().fbh_shap_model_create(0, 1, N.ptr(offs), *(N.ptr(v) for v in a.values()),
+                                              None, None, None, 0, D, 0.0, C.byref(h)))
+    x = np.ones((65, D), np.float32)
+    x[0] = -1.0        # down the whole path
+    x[1, :7] = -1.0    # to its last right leaf
+    x[2, ::2] = -1.0
+    try:
+        out = {}
+        for order in (0, 1):
+            out[order] = np.full((65, D + 1), np.nan, np.float32)
+            N.check_hip(N.hip().fbh_shap_set_host_order(h, order))
+            N.check_hip(N.hip().fbh_shap_contribs(h, N.ptr(x), 65, None, N.ptr(out[order])))
+        if not fits:
+            assert np.array_equal(out[0], out[1], equal_nan=True)
+            return
+        margin = np.zeros(65, np.float32)
+        N.check_hip(N.hip().fbh_predict(h, N.ptr(x), 65, None, 0, N.ptr(margin)))
+        # (the weights sum to 1 + share at each node, not to 1: rows add up to within
+        # the covers' own error)
+        assert np.isfinite(out[0]).all()
+        assert np.max(np.abs(out[0].sum(1) - margin)) <= 16 * share + 8 * 16 * 2.0 ** -24
+    finally:
+        N.hip().fbh_shap_model_destroy(h)
