@@ -676,6 +676,7 @@ constexpr uint32_t PRED_LDS_BYTES = 160 * 1024, PRED_LEAFV_BYTES = 8 * 1024;
 constexpr uint32_t PRED_TILES_MAX_F = 500;  // features of which 64 rows fit beside 2,500 nodes
 constexpr uint32_t PRED_FILL_TILES = 256;   // workgroups that fill the device
 constexpr uint64_t PRED_WORK_BYTES = 64ull << 20;  // most of a split call's leaf values
+constexpr uint32_t PRED_LDS4_MAX_F = 255;  // features whose rows predict_lds4_kernel holds in LDS
 
 struct PredRun {
     uint32_t tree0, n_trees;
@@ -689,10 +690,13 @@ struct PredTrees {
     uint32_t n_trees, n_runs, n_features;
     uint32_t groups;            // groups of 64 rows a workgroup can hold: 1, 2 or 4
     uint32_t most_nodes;        // of a run
+    uint64_t n_entries;         // of all runs
 };
 // Device bytes of the leaf values a call of so few rows that its runs are split
 // over workgroups goes through (0: none).
 uint64_t predict_tiles_work(const PredTrees &P, uint64_t n_rows, uint32_t mode);
+// Whether that is faster than walking the nodes in memory.
+bool predict_tiles_pay(const PredTrees &P, uint64_t n_rows, uint32_t mode);
 // Margins, values (PRED_OUT_SIGMOID) or leaf ids; `work` of
 // predict_tiles_work's bytes, or null.
 hipError_t launch_predict_tiles(const PredTrees &P, const float *rows, uint64_t n_rows,

@@ -33,6 +33,7 @@
 #include "fb_expf.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace fbh {
 
@@ -294,20 +295,15 @@ hipError_t launch_groups(uint32_t g, const PredTrees &P, uint32_t split, const f
     return launch_tile<1, CATS>(P, split, rows, n, init, base, mode, vals, out, s);
 }
 
-}  // namespace
-
-uint64_t predict_tiles_work(const PredTrees &P, uint64_t n_rows, uint32_t mode) {
+// The groups of 64 rows a workgroup takes, and the workgroups that share the runs of
+// its rows.
+struct TileShape {
+    uint32_t groups, split;
+};
+TileShape tile_shape(const PredTrees &P, uint64_t n_rows, uint32_t mode, bool work) {
     const uint64_t tiles = (n_rows + 63) / 64;
-    if (mode > PRED_OUT_SIGMOID || P.n_runs < 2 || tiles >= PRED_FILL_TILES) return 0;
-    const uint64_t bytes = 4 * n_rows * P.n_trees;
-    return bytes <= PRED_WORK_BYTES ? bytes : 0;
-}
-
-hipError_t launch_predict_tiles(const PredTrees &P, const float *rows, uint64_t n_rows,
-                                const float *init, float base, uint32_t mode, float *out,
-                                void *work, hipStream_t s) {
-    if (n_rows == 0) return hipSuccess;
-    const uint64_t tiles = (n_rows + 63) / 64;
+    if (work || (mode == PRED_OUT_LEAF && tiles < PRED_FILL_TILES))
+        return {1, (uint32_t)std::min<uint64_t>(P.n_runs, (PRED_FILL_TILES + tiles - 1) / tiles)};
     // More groups of 64 rows a workgroup read the trees fewer times; fewer leave
     // less of the device idle in the last round of tiles. The most groups within
     // a tenth of the least rounds' rows.
@@ -319,11 +315,61 @@ hipError_t launch_predict_tiles(const PredTrees &P, const float *rows, uint64_t 
         if (rounds * 10 <= least * 11 || least == ~0ull) g = k;
         least = std::min(least, rounds);
     }
-    uint32_t split = 1;
-    if (work || (mode == PRED_OUT_LEAF && tiles < PRED_FILL_TILES)) {
-        g = 1;
-        split = (uint32_t)std::min<uint64_t>(P.n_runs, (PRED_FILL_TILES + tiles - 1) / tiles);
+    return {g, 1};
+}
+
+}  // namespace
+
+uint64_t predict_tiles_work(const PredTrees &P, uint64_t n_rows, uint32_t mode) {
+    const uint64_t tiles = (n_rows + 63) / 64;
+    if (mode > PRED_OUT_SIGMOID || P.n_runs < 2 || tiles >= PRED_FILL_TILES) return 0;
+    const uint64_t bytes = 4 * n_rows * P.n_trees;
+    return bytes <= PRED_WORK_BYTES ? bytes : 0;
+}
+
+// Estimates in microseconds. Here a CU takes 2.6 to 4 for a run of trees, whether 16
+// waves share 32 small trees or one walks a tree that fills the run, and no less than
+// its rows take to arrive. The walks that read the nodes from memory take a time for
+// each (tree, 64 rows), longer for deeper trees and, up to 255 features, for the
+// fewer workgroups whose rows fit a CU; few rows wait for one tree after the other.
+// Measured (200k rows, here against there): 28 features, 8 runs of 1, 5 and 12 trees
+// 229, 239, 247 against 68, 149, 258 us; 200 features 401, 395, 419 against 199, 426,
+// 711; 400 features, where the other walk reads rows in place, 8 runs of 1 and 2 trees
+// 452, 443 against 352, 616, and one run of 1 and 8 trees of 63 nodes 139 against 32
+// and 160. Of 201 such measurements (1k to 200k rows, 63 to 12,783 nodes a tree) the
+// rule takes a walk more than 7 % slower than the other in three, 16 % at most.
+bool predict_tiles_pay(const PredTrees &P, uint64_t n_rows, uint32_t mode) {
+    const bool work = predict_tiles_work(P, n_rows, mode) != 0;
+    const TileShape shape = tile_shape(P, n_rows, mode, work);
+    const double tiles = (double)((n_rows + 63) / 64), nf = P.n_features, trees = P.n_trees;
+    const uint64_t blocks = ((n_rows + 63) / 64 + shape.groups - 1) / shape.groups * shape.split;
+    const double rounds = (double)((blocks + PRED_CUS - 1) / PRED_CUS);
+    const uint32_t runs = (P.n_runs + shape.split - 1) / shape.split;
+    const bool in_lds = P.n_features <= PRED_LDS4_MAX_F;
+    if (in_lds && rounds == 1 && runs == 1) return true;
+    const double fill = std::min(1.0, (double)P.n_entries / P.n_runs / PRED_RUN_NODES);
+    const double rows_us = in_lds ? 0.011 * nf * shape.groups : 0.0235 * nf;
+    const double here = rounds * std::max(runs * (2.6 + 1.4 * fill), rows_us + 0.9) + (work ? 2 : 0);
+    const double depth = std::log2(P.n_entries / trees + 1);
+    double there;
+    if (in_lds) {
+        const uint32_t held = std::min(8u, PRED_LDS_BYTES / (256 * ((P.n_features | 1u) + 32)));
+        const double each = (0.45 + 5.2 / held) * std::pow(depth / 13.6, 1.5);
+        there = std::max(tiles * ((0.11 + 0.0005 * nf) * nf + trees * each) * 1e-3,
+                         trees * 0.05 * depth);
+    } else {
+        there = std::max(tiles * trees * std::min(10.5, depth) * 1e-3, trees * 0.25 * depth);
     }
+    return here <= 1.05 * there;
+}
+
+hipError_t launch_predict_tiles(const PredTrees &P, const float *rows, uint64_t n_rows,
+                                const float *init, float base, uint32_t mode, float *out,
+                                void *work, hipStream_t s) {
+    if (n_rows == 0) return hipSuccess;
+    const uint64_t tiles = (n_rows + 63) / 64;
+    const TileShape shape = tile_shape(P, n_rows, mode, work != nullptr);
+    const uint32_t g = shape.groups, split = shape.split;
     const uint32_t mk = work ? PRED_OUT_VALUES : mode;
     float *vals = static_cast<float *>(work);
     hipError_t e = P.categorical

@@ -155,8 +155,8 @@ __global__ __launch_bounds__(PRED_TPB) void predict_kernel(
 
 constexpr uint32_t PRED_LDS_ROWS = 64;
 
-// The same walk, for models with a tree too large for fbhip_predict.hip, over
-// 64 rows copied into LDS (coalesced loads; row stride nf | 1, odd, so the 64
+// The same walk, for models with a tree too large for fbhip_predict.hip and where
+// that one does not pay (predict_tiles_pay), over 64 rows copied into LDS (coalesced loads; row stride nf | 1, odd, so the 64
 // lanes' cells of one feature fall in distinct banks) and shared by four
 // waves, which take every fourth tree of a run of PRED_RUN trees and put each
 // row's leaf value in LDS; wave 0 then adds the run's values to the row's
@@ -164,7 +164,8 @@ constexpr uint32_t PRED_LDS_ROWS = 64;
 // bit-identical), and the waves go on to the next run.
 constexpr uint32_t PRED_WAVES = 4;
 constexpr uint32_t PRED_RUN = 32;
-constexpr uint32_t PRED_LDS4_MAX_F = 223;  // 64 x 224 + 64 x 32 floats: 64 KiB of LDS
+// Up to PRED_LDS4_MAX_F features, 72 KiB of LDS: two workgroups a CU. 200k rows of 230
+// features, 128 trees of 511 nodes and one of 16,383: 868 us, read in place 3,138.
 
 __global__ __launch_bounds__(PRED_LDS_ROWS * PRED_WAVES) void predict_lds4_kernel(
     const PredNodeDev *__restrict__ nodes, const ShapNodeDev *__restrict__ full,
@@ -1205,6 +1206,10 @@ void check_kind(const fbh_shap_model *m, Kind k) {
     }
 }
 
+uint32_t pred_mode(Kind k) {
+    return k == Kind::Leaf ? PRED_LEAF : k == Kind::Value ? PRED_SIGMOID : PRED_MARGIN;
+}
+
 // Enqueues one kind over device-resident rows on the model's stream.
 void enqueue(fbh_shap_model *m, Kind k, const float *d_rows, uint64_t n, const float *d_margin,
              float *d_out) {
@@ -1227,19 +1232,22 @@ void enqueue(fbh_shap_model *m, Kind k, const float *d_rows, uint64_t n, const f
             chk(hipGetLastError(), "saabas launch");
             return;
         default: {
-            const uint32_t mode = k == Kind::Leaf ? PRED_LEAF
-                                  : k == Kind::Value ? PRED_SIGMOID : PRED_MARGIN;
+            const uint32_t mode = pred_mode(k);
             const uint32_t nf = m->n_features;
-            if (m->pred.nodes) {
+            if (m->pred.nodes && predict_tiles_pay(m->pred, n, mode)) {
                 run_predict(m, d_rows, n, d_margin, mode, d_out);
                 return;
             }
             if (nf >= 1 && nf <= PRED_LDS4_MAX_F) {
                 const uint32_t lb = (uint32_t)((n + PRED_LDS_ROWS - 1) / PRED_LDS_ROWS);
+                const size_t lds = (size_t)PRED_LDS_ROWS * ((nf | 1u) + PRED_RUN) * 4;
+                if (lds > 64 * 1024)
+                    chk(hipFuncSetAttribute(reinterpret_cast<const void *>(&predict_lds4_kernel),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
+                        "predict LDS");
                 hipLaunchKernelGGL(predict_lds4_kernel, dim3(lb), dim3(PRED_LDS_ROWS * PRED_WAVES),
-                                   (size_t)PRED_LDS_ROWS * ((nf | 1u) + PRED_RUN) * 4, m->stream,
-                                   m->d_pred, m->d_nodes, m->d_cats, m->d_roots, m->n_trees,
-                                   d_rows, n, nf, d_margin, m->bias, mode, d_out);
+                                   lds, m->stream, m->d_pred, m->d_nodes, m->d_cats, m->d_roots,
+                                   m->n_trees, d_rows, n, nf, d_margin, m->bias, mode, d_out);
             } else {
                 hipLaunchKernelGGL(predict_kernel, dim3(blocks), dim3(PRED_TPB), 0, m->stream,
                                    m->d_pred, m->d_nodes, m->d_cats, m->d_roots, m->n_trees, d_rows,
@@ -1302,9 +1310,10 @@ uint64_t round256(uint64_t v) { return (v + 255) & ~uint64_t(255); }
 
 // Whether the kind's kernels read a row a few times in order and write each
 // output once.
-bool runs_in_place(const fbh_shap_model *m, Kind k) {
+bool runs_in_place(const fbh_shap_model *m, Kind k, uint64_t n) {
     if (k == Kind::Contribs) return takes_paths(m, false);
-    return (k == Kind::Margin || k == Kind::Value || k == Kind::Leaf) && m->pred.nodes;
+    if ((k != Kind::Margin && k != Kind::Value && k != Kind::Leaf) || !m->pred.nodes) return false;
+    return m->n_features <= PRED_LDS4_MAX_F || predict_tiles_pay(m->pred, n, pred_mode(k));
 }
 
 // Host call: batches of at most 512 MiB of inputs and outputs
@@ -1320,7 +1329,7 @@ void run_host_alloc(fbh_shap_model *m, Kind k, const float *rows, uint64_t n_row
     const uint64_t w = out_width(m, k), nf = m->n_features;
     const uint64_t per_row = 4ull * (nf + 1 + w);
     std::unique_lock<std::mutex> mine(m->host_mu, std::try_to_lock);
-    if (mine && n_rows <= PINNED_BYTES / per_row && runs_in_place(m, k)) {
+    if (mine && n_rows <= PINNED_BYTES / per_row && runs_in_place(m, k, n_rows)) {
         if (!m->pinned) chk(keep_alloc(KeepKind::host, &m->pinned, PINNED_BYTES + 1024), "pinned");
         float *x = static_cast<float *>(m->pinned);
         float *mg = x + round256(4 * n_rows * nf) / 4, *o = mg + round256(4 * n_rows) / 4;
@@ -1668,6 +1677,7 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
             q.n_features = n_features;
             q.groups = pt.groups;
             q.most_nodes = pt.most_nodes;
+            for (const PredRun &r : pt.runs) q.n_entries += r.n_nodes;
             arrays.add(pt.nodes, q.nodes);
         }
         if (pb.ok && !pb.nodes.empty() && m->cover_error.empty()) {

@@ -76,3 +76,19 @@ def test_margins_and_leaf_ids(lib, rows, n_trees, depth, nf, n_cat, full):  # no
         assert np.array_equal(leaf, ids)
     finally:
         N.hip().fbh_shap_model_destroy(h)
+
+
+@pytest.mark.parametrize("rows,n_trees,depth,nf,n_cat,full", [
+    (20_000, 3, 12, 28, 3, True),    # a tree a run: walked from memory, rows in LDS
+    (20_000, 6, 11, 40, 0, True),    # three trees a run: likewise
+    (1_000, 3, 12, 28, 3, True),     # few rows: the runs split over workgroups
+    (40_000, 1, 2, 28, 0, True),     # one small tree
+    (33_000, 2, 5, 400, 5, True),    # two small trees of wide rows: read in place
+    (500, 2, 13, 240, 3, True),      # trees larger than a run, rows past 64 KiB of LDS
+    (130, 2, 13, 255, 0, True),      # the widest of those
+    (130, 2, 13, 256, 3, True),      # wider: read in place
+])
+def test_large_and_few_trees(lib, rows, n_trees, depth, nf, n_cat, full):  # noqa: F811
+    """Both sides of predict_tiles_pay, and of the row widths of the walk it leaves
+    the others to."""
+    test_margins_and_leaf_ids(lib, rows, n_trees, depth, nf, n_cat, full)
