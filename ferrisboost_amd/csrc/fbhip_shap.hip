@@ -29,6 +29,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <future>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -810,25 +811,45 @@ struct fbh_shap_model {
         return e;
     }
     uint64_t held_bytes() const { return array_bytes + work_bytes + staging_bytes; }
-    // The arrays added so far, laid out in one allocation and sent in one copy.
+    // Arrays of one allocation: sent in one copy where they are small (a copy takes
+    // about 10 us however few its bytes), each from its own place where gathering
+    // them would take longer.
     struct Arrays {
-        std::vector<unsigned char> bytes;
-        std::vector<std::function<void(unsigned char *)>> place;
+        static constexpr size_t GATHER_MOST = 2 << 20;
+        struct Part {
+            const void *from;
+            size_t bytes, off;
+            std::function<void(unsigned char *)> place;
+        };
+        std::vector<Part> parts;
+        size_t bytes = 0;
         template <class T, class P>
         void add(const std::vector<T> &v, P *&to) {
-            const size_t off = (bytes.size() + 255) & ~size_t(255);
-            bytes.resize(off + std::max<size_t>(sizeof(T) * v.size(), 64));
-            if (!v.empty()) std::memcpy(bytes.data() + off, v.data(), sizeof(T) * v.size());
-            place.push_back([&to, off](unsigned char *base) { to = reinterpret_cast<P *>(base + off); });
+            const size_t off = (bytes + 255) & ~size_t(255);
+            parts.push_back({v.data(), sizeof(T) * v.size(), off, [&to, off](unsigned char *base) {
+                                 to = reinterpret_cast<P *>(base + off);
+                             }});
+            bytes = off + std::max<size_t>(sizeof(T) * v.size(), 64);
         }
     };
     void upload(const Arrays &a) {
         void *p = nullptr;
-        chk(keep_alloc(KeepKind::device, &p, a.bytes.size()), "model arrays");
+        chk(keep_alloc(KeepKind::device, &p, a.bytes), "model arrays");
         allocs.push_back(p);
-        array_bytes += a.bytes.size();
-        chk(hipMemcpy(p, a.bytes.data(), a.bytes.size(), hipMemcpyHostToDevice), "model arrays");
-        for (const auto &f : a.place) f(static_cast<unsigned char *>(p));
+        array_bytes += a.bytes;
+        unsigned char *base = static_cast<unsigned char *>(p);
+        if (a.bytes <= Arrays::GATHER_MOST) {
+            std::vector<unsigned char> all(a.bytes);
+            for (const Arrays::Part &part : a.parts)
+                if (part.bytes) std::memcpy(all.data() + part.off, part.from, part.bytes);
+            chk(hipMemcpy(p, all.data(), a.bytes, hipMemcpyHostToDevice), "model arrays");
+        } else {
+            for (const Arrays::Part &part : a.parts)
+                if (part.bytes)
+                    chk(hipMemcpy(base + part.off, part.from, part.bytes, hipMemcpyHostToDevice),
+                        "model arrays");
+        }
+        for (const Arrays::Part &part : a.parts) part.place(base);
     }
 };
 
@@ -891,45 +912,42 @@ struct PathBuild {
     bool ok = true;
 
     void add_tree(const std::vector<ShapNodeDev> &n, uint32_t root) {
-        std::vector<Edge> path;
-        if (ok && !(n[root].flags & 1u)) add(n, root, path, 1.0);
+        if (ok && !(n[root].flags & 1u)) add(n, root, 0, 0, 1.0);
         first.push_back((uint32_t)nodes.size());
     }
 
 private:
-    // an edge of the path: its feature, and the product of the weights of that
-    // feature's edges down to it
-    struct Edge {
-        uint32_t feat;
-        double z;
-    };
+    // The path's edges: the feature, and the product of the weights of that feature's
+    // edges down to it.
+    uint32_t feats_[SHAP_PATHS_DEPTH];
+    double z_[SHAP_PATHS_DEPTH];
 
-    void add(const std::vector<ShapNodeDev> &n, uint32_t id, std::vector<Edge> &path, double weight) {
+    // The node at `depth` edges below the root, of which `newest` (a bit a depth) are
+    // their feature's newest, with the product of their weights.
+    void add(const std::vector<ShapNodeDev> &n, uint32_t id, int depth, uint32_t newest,
+             double weight) {
         const ShapNodeDev &d = n[id];
-        const int depth = (int)path.size();
         if (depth >= SHAP_PATHS_DEPTH) ok = false;
         if (!ok) return;
-        PathNodeDev p{};
-        PathTestDev t{};
+        tests.emplace_back();
+        PathTestDev &t = tests.back();
         t.ff = d.feat | ((d.flags & 2u) ? PATH_DEFAULT_LEFT : 0u) | ((d.flags & 4u) ? PATH_CAT : 0u);
         t.cond = d.split_cond;
         t.cat_offset = d.cat_offset;
         t.cat_len = d.cat_len;
         if (!(d.flags & 4u) && std::isnan(d.split_cond)) ok = false;
-        p.meta = d.feat << PATH_FEATURE;
+        nodes.emplace_back();
+        PathNodeDev &p = nodes.back();
+        uint32_t meta = d.feat << PATH_FEATURE;
         double older = 1.0;
-        for (int k = depth - 1; k >= 0; k--) {
-            if (path[k].feat == d.feat) {
-                if (!(p.meta & PATH_AGAIN)) {
-                    p.meta |= PATH_AGAIN | (uint32_t)k << PATH_OLDER;
-                    older = path[k].z;
-                }
-                continue;
+        for (uint32_t k = 0; k < (uint32_t)depth; k++)
+            if ((newest >> k & 1u) && feats_[k] == d.feat) {
+                meta |= PATH_AGAIN | k << PATH_OLDER;
+                older = z_[k];
+                newest &= ~(1u << k);
+                break;
             }
-            bool newest = true;
-            for (int j = k + 1; j < depth; j++) newest &= path[j].feat != path[k].feat;
-            if (newest) p.meta |= 1u << (PATH_PARTNERS + k);
-        }
+        meta |= newest << PATH_PARTNERS;
         const uint32_t child[2] = {(uint32_t)d.left, (uint32_t)d.right};
         const double w[2] = {(double)d.left_weight, (double)d.right_weight};
         float a[2], v[2] = {0.0f, 0.0f};
@@ -944,23 +962,22 @@ private:
                 if (weight * w[s] < 1e-36) ok = false;
                 continue;
             }
-            p.meta |= s ? PATH_LEAF_R : PATH_LEAF_L;
+            meta |= s ? PATH_LEAF_R : PATH_LEAF_L;
             const double leaf = (double)c.leaf_value * weight * w[s];
             v[s] = (float)leaf;
             if (!std::isfinite(leaf) || (leaf != 0.0 && std::fabs(leaf) < 1e-36)) ok = false;
         }
+        p.meta = meta;
         p.al = a[0];
         p.ar = a[1];
         p.vl = v[0];
         p.vr = v[1];
         p.s0 = v[0] + v[1];
-        nodes.push_back(p);
-        tests.push_back(t);
+        feats_[depth] = d.feat;
         for (int s = 0; s < 2; s++) {
             if (n[child[s]].flags & 1u) continue;
-            path.push_back({d.feat, older * w[s]});
-            add(n, child[s], path, weight * w[s]);
-            path.pop_back();
+            z_[depth] = older * w[s];
+            add(n, child[s], depth + 1, newest | 1u << depth, weight * w[s]);
         }
     }
 };
@@ -975,6 +992,7 @@ struct PredBuild {
     bool ok = true, categorical = false;
     uint32_t done = 0;  // trees
     uint32_t groups = 1, cap = 0, trees = PRED_RUN_TREES, most_nodes = 0;
+    std::vector<uint32_t> order_;
 
     // The rows a workgroup holds, a run's most entries beside them, and its most
     // trees such that the runs are of a size.
@@ -1014,33 +1032,44 @@ struct PredBuild {
     void add_tree(const std::vector<ShapNodeDev> &n, uint32_t root, uint32_t count,
                   const uint32_t *cat_words) {
         if (!ok) return;
-        std::vector<uint32_t> order{root};
+        order_.resize(count);
+        uint32_t *const order = order_.data();
+        order[0] = root;
+        uint32_t n_order = 1;
         uint64_t words = 0;
-        for (uint32_t i = 0; i < order.size() && order.size() <= count; i++) {
+        for (uint32_t i = 0; i < n_order; i++) {
             const ShapNodeDev &d = n[order[i]];
             if (d.flags & 1u) continue;
             words += d.cat_len;
-            order.push_back((uint32_t)d.left);
-            order.push_back((uint32_t)d.right);
+            if (n_order + 2 > count) {  // a node under two parents
+                ok = false;
+                return;
+            }
+            order[n_order++] = (uint32_t)d.left;
+            order[n_order++] = (uint32_t)d.right;
         }
-        const uint64_t size = order.size() + (words + 1) / 2;
-        if (order.size() > count || HEAD + size > cap) {  // a node under two parents, or too large
+        const uint64_t size = n_order + (words + 1) / 2;
+        if (HEAD + size > cap) {
             ok = false;
             return;
         }
         if (runs.empty() || runs.back().n_trees == trees || runs.back().n_nodes + size > cap) {
             if (nodes.size() & 1) nodes.push_back(make_uint2(0, 0));  // loaded two at a time
             runs.push_back({done, 0, (uint32_t)nodes.size(), HEAD});
-            nodes.resize(nodes.size() + HEAD);
+            nodes.resize(nodes.size() + HEAD, make_uint2(0, 0));
         }
         PredRun &run = runs.back();
         uint2 &first = nodes[run.node0 + run.n_trees / 2];
         (run.n_trees & 1 ? first.y : first.x) = run.n_nodes;
         done++;
-        ids.resize(nodes.size());
-        std::vector<uint32_t> set;
-        uint32_t child = 1;
-        for (uint32_t i = 0; i < order.size(); i++) {
+        const size_t at = nodes.size();
+        nodes.resize(at + size, make_uint2(0, 0));
+        ids.resize(at + n_order);
+        uint2 *const to = nodes.data() + at;
+        uint32_t *const set = reinterpret_cast<uint32_t *>(to + n_order);
+        uint32_t *const id = ids.data() + at;
+        uint32_t child = 1, in_set = 0;
+        for (uint32_t i = 0; i < n_order; i++) {
             const ShapNodeDev &d = n[order[i]];
             uint2 p;
             if (d.flags & 1u) {
@@ -1054,18 +1083,15 @@ struct PredBuild {
                 if (d.flags & 4u) {
                     categorical = true;
                     p.y |= PRED_CAT_BIT;
-                    p.x = (2 * (run.n_nodes + (uint32_t)order.size()) + (uint32_t)set.size()) |
-                          d.cat_len << 16;
-                    set.insert(set.end(), cat_words + d.cat_offset,
-                               cat_words + d.cat_offset + d.cat_len);
+                    p.x = (2 * (run.n_nodes + n_order) + in_set) | d.cat_len << 16;
+                    std::memcpy(set + in_set, cat_words + d.cat_offset, 4 * d.cat_len);
+                    in_set += d.cat_len;
                 }
                 child += 2;
             }
-            nodes.push_back(p);
-            ids.push_back(order[i] - root);
+            to[i] = p;
+            id[i] = order[i] - root;
         }
-        for (size_t k = 0; k < set.size(); k += 2)
-            nodes.push_back(make_uint2(set[k], k + 1 < set.size() ? set[k + 1] : 0u));
         run.n_trees++;
         run.n_nodes += (uint32_t)size;
         most_nodes = std::max(most_nodes, run.n_nodes);
@@ -1561,9 +1587,6 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         std::vector<float> means(total, 0.0f);
         std::vector<uint32_t> roots(n_trees), uoff(n_trees + 1, 0), ufeats;
         double rm_sum = 0.0;
-        PathBuild pb;
-        pb.ok = n_features <= SHAP_PATHS_MAX_F;
-        PredBuild pt(n_features, tree_offsets, n_trees, cat_len);
         for (uint32_t t = 0; t < n_trees; t++) {
             const uint32_t b = tree_offsets[t], e = tree_offsets[t + 1];
             if (e <= b) throw ShapError(FBH_INPUT_ERROR, "tree " + std::to_string(t) + " has no nodes");
@@ -1640,8 +1663,6 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
                 throw ShapError(FBH_INPUT_ERROR, "a tree splits on more than " +
                                                      std::to_string(MAX_SHAP_UNIQUE) +
                                                      " distinct features");
-            pb.add_tree(nodes, b);
-            pt.add_tree(nodes, b, e - b, cat_words);
             rm_sum += root_mean(L, R, lv, hs, lf, b, 0);
             node_means(L, R, lv, hs, lf, b, 0, means);
         }
@@ -1656,6 +1677,23 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         m->n_nodes = total;
         m->bias = bias;
         m->root_mean = (float)rm_sum;
+        PathBuild pb;
+        pb.ok = n_features <= SHAP_PATHS_MAX_F && m->cover_error.empty();
+        PredBuild pt(n_features, tree_offsets, n_trees, cat_len);
+        auto make_paths = [&] {
+            if (!pb.ok) return;
+            pb.nodes.reserve(total / 2 + 2);
+            pb.tests.reserve(total / 2 + 9);
+            for (uint32_t t = 0; t < n_trees; t++) pb.add_tree(nodes, tree_offsets[t]);
+        };
+        auto make_runs = [&] {
+            if (!pt.ok) return;
+            const size_t n = total + (n_trees / pt.trees + 2) * (PredBuild::HEAD + 1);
+            pt.nodes.reserve(n);
+            pt.ids.reserve(n);
+            for (uint32_t t = 0; t < n_trees; t++)
+                pt.add_tree(nodes, tree_offsets[t], tree_offsets[t + 1] - tree_offsets[t], cat_words);
+        };
         fbh_shap_model::Arrays arrays;
         arrays.add(nodes, m->d_nodes);
         arrays.add(rec, m->d_rec);
@@ -1666,8 +1704,24 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         arrays.add(ufeats, m->d_ufeats);
         arrays.add(cw, m->d_cats);
         arrays.add(rv, m->d_rule);
+        // Of a model worth two threads, the records of the kernels of this file are
+        // sent while those of the others are made, so that the first call on a model
+        // waits little longer than for these alone: 200 trees of depth 8 3.3 ms, 3.9
+        // on one thread, 2.9 without the others; 100 trees 1.5, 1.3 and 1.0.
+        constexpr uint32_t THREADS_LEAST = 1 << 16;  // nodes
+        if (total >= THREADS_LEAST) {
+            auto paths = std::async(std::launch::async, make_paths);
+            auto runs = std::async(std::launch::async, make_runs);
+            m->upload(arrays);
+            arrays = {};
+            paths.get();
+            runs.get();
+        } else {
+            make_paths();
+            make_runs();
+        }
         if (pt.ok && n_trees) {
-            pt.nodes.resize(pt.nodes.size() + 1);  // a run's last pair may be half
+            pt.nodes.push_back(make_uint2(0, 0));  // a run's last pair may be half
             PredTrees &q = m->pred;
             arrays.add(pt.runs, q.runs);
             arrays.add(pt.ids, q.ids);
@@ -1680,7 +1734,7 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
             for (const PredRun &r : pt.runs) q.n_entries += r.n_nodes;
             arrays.add(pt.nodes, q.nodes);
         }
-        if (pb.ok && !pb.nodes.empty() && m->cover_error.empty()) {
+        if (pb.ok && !pb.nodes.empty()) {
             uint32_t most = 0;
             for (uint32_t t = 0; t < n_trees; t++) most = std::max(most, pb.first[t + 1] - pb.first[t]);
             // the walk requests one node past a tree's last, the tests are read
@@ -1690,7 +1744,6 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
             ShapPaths &q = m->paths;
             arrays.add(pb.tests, q.tests);
             arrays.add(pb.first, q.first);
-            arrays.add(cw, q.cats);
             q.n_trees = n_trees;
             q.n_features = n_features;
             q.stride = (most + 8) & ~7u;
@@ -1700,7 +1753,8 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
             q.root_mean = m->root_mean;
             arrays.add(pb.nodes, q.nodes);
         }
-        m->upload(arrays);
+        if (arrays.bytes) m->upload(arrays);
+        m->paths.cats = m->d_cats;
         *out = m.release();
     });
 }
