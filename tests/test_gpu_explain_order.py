@@ -84,3 +84,18 @@ def test_the_order_applies_to_treeshap_alone(models):
                {"pred_contribs": True, "approx_contribs": True}):
         with pytest.raises(ValueError, match="engine_order"):
             m.predict(x, engine_order=True, **kw)
+
+
+@pytest.mark.parametrize("nf,rows", [(63, 63), (63, 64), (64, 65), (511, 8), (512, 8), (300, 9)])
+def test_wide_rows_on_both_sides_of_the_copies(nf, rows):
+    """Contributions of rows read over the link and of rows copied first (32 KiB of 64
+    rows in and out is where they part): the same bits as in a batch of 700."""
+    import ferrisboost_amd as fb
+
+    rng = np.random.default_rng(nf)
+    x = rng.normal(size=(ROWS, nf)).astype(np.float32)
+    m = fb.train({"max_depth": 4, "objective": "reg:squarederror"}, x, x[:, 0] * x[:, 1],
+                 num_boost_round=5)
+    whole = m.predict(x, pred_contribs=True)
+    part = m.predict(x[:rows], pred_contribs=True)
+    assert np.array_equal(part.view(np.uint32), whole[:rows].view(np.uint32))
