@@ -94,14 +94,7 @@ constexpr uint32_t SK_FEATS = 64;  // features of a staging tile
 constexpr uint32_t SK_MAX_BIN = 1024;                   // largest max_bin sketched here
 constexpr uint64_t SK_STAGE_BYTES = 256ull << 20;      // row staging of one chunk
 constexpr uint64_t KEEP_CHUNK_BYTES = 64ull << 20;     // rows uploaded, then sketched, at a time
-// Features are summarised in groups that share the summary buffers, of GROUP_BYTES of
-// batch summaries but no fewer than GROUP_FEATS features: a merge of each still gives
-// every CU a workgroup at the counter's last levels. 400k x 2000 at 256 bins takes 33
-// GB in one group, more than is kept for the next job (fbhip_keep.hip), and 11 in groups:
-// the whole job, 40 rounds, 239 -> 226 ms, and 221 with a group's task tables
-// built while the groups before it run.
-constexpr uint32_t GROUP_FEATS = 256;
-constexpr uint64_t GROUP_BYTES = 2ull << 30;
+static_assert(sizeof(SkEntry) == SKETCH_ENTRY_BYTES, "a summary entry");
 
 __host__ __device__ inline uint32_t sk_limit(uint32_t max_bin) {
     const uint32_t l = 16u * max_bin;
@@ -719,18 +712,25 @@ __global__ __launch_bounds__(SK_TPB) void sk_cuts_kernel(const SkCutTask *__rest
     if (threadIdx.x == 0) *T.n_out = kept;
 }
 
-uint32_t bit_length(uint64_t v) {
-    uint32_t b = 0;
-    while (v) {
-        b++;
-        v >>= 1;
-    }
-    return b;
-}
-
 uint64_t stage_rows_of(uint64_t n_rows, uint32_t nf) {
     const uint64_t r = std::max<uint64_t>(SK_ROWS, SK_STAGE_BYTES / (4ull * std::max(nf, 1u)));
     return std::max<uint64_t>(1, std::min(n_rows, r));
+}
+
+// Bytes of the task tables: at most a pruning merge a batch, and fewer final merges
+// than slots for them.
+uint64_t task_bytes(const SketchSlots &k, uint32_t n_num) {
+    return sizeof(SkSortTask) * k.all_a + sizeof(SkMergeTask) * (k.all_a + k.all_t) +
+           sizeof(SkCutTask) * (uint64_t)n_num;
+}
+
+// Device bytes of the summaries, cuts and task tables (fbh_sketch_cuts).
+uint64_t summary_bytes(const SketchSlots &k, uint32_t n_num, uint32_t max_bin) {
+    const uint64_t L = sk_limit(max_bin);
+    return SKETCH_ENTRY_BYTES * L * (k.a + 2 * k.b + k.t + n_num)  // levels, finals, compressed
+           + 4 * (k.a + k.b + k.t)                                 // entry counts
+           + 4ull * n_num * max_bin                                // cuts and their counts
+           + task_bytes(k, n_num);
 }
 
 // Device bytes of the sketch, with every value of every numeric feature
@@ -742,15 +742,7 @@ uint64_t sketch_bytes(uint64_t n_rows, uint32_t nf, uint32_t n_num, uint32_t max
     b += 4 * n_rows * n_num;  // compacted values
     if (max_bin >= 2) {
         const uint64_t L = sk_limit(max_bin);
-        const uint64_t m = (n_rows + L - 1) / L;  // batches of a feature
-        const uint64_t per = 16 * m * L                   // level buffer A
-                             + 16 * ((m + 1) / 2) * 2 * L  // level buffer B
-                             + 16 * 2 * bit_length(m) * L  // final merges
-                             + 16 * L                       // compressed summary
-                             + 8 * (m + 1)                  // entry counts
-                             + sizeof(SkSortTask) * m + sizeof(SkMergeTask) * (m + bit_length(m)) +
-                             sizeof(SkCutTask) + 4 * max_bin + 64;
-        b += per * n_num;
+        b += summary_bytes(sketch_slots_most((n_rows + L - 1) / L, n_num, L), n_num, max_bin);
     }
     return b;
 }
@@ -1109,32 +1101,14 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
         const uint32_t max_bin = s->max_bin;
         const uint32_t n_cuts = max_bin >= 1 ? max_bin - 1 : 0;
         const uint64_t L = sk_limit(max_bin);
-        std::vector<uint64_t> m(nn, 0), abase(nn + 1, 0), bbase(nn + 1, 0), tbase(nn + 1, 0);
-        for (uint32_t j = 0; j < nn; j++) {
-            m[j] = n_cuts ? (n_valid[j] + L - 1) / L : 0;
-            abase[j + 1] = abase[j] + m[j];
-            bbase[j + 1] = bbase[j] + (m[j] + 1) / 2;
-            tbase[j + 1] = tbase[j] + (m[j] ? 2ull * __builtin_popcountll(m[j]) : 0ull);
-        }
+        std::vector<uint64_t> m(nn, 0);
+        for (uint32_t j = 0; j < nn; j++) m[j] = n_cuts ? (n_valid[j] + L - 1) / L : 0;
+        const SketchPlan plan = sketch_plan(m, L);
+        const std::vector<uint64_t> &abase = plan.abase, &bbase = plan.bbase, &tbase = plan.tbase;
         std::vector<uint32_t> n_out(nn, 0);
         std::vector<float> cuts_dev;
         if (abase[nn]) {
-            struct Group {
-                uint32_t j0, j1;
-            };
-            std::vector<Group> groups;
-            uint64_t na = 0, nb = 0, nt = 0;  // the largest group's slots
-            for (uint32_t j0 = 0, j1; j0 < nn; j0 = j1) {
-                j1 = j0 + 1;
-                while (j1 < nn && (j1 - j0 < GROUP_FEATS ||
-                                   (abase[j1 + 1] - abase[j0]) * L * sizeof(SkEntry) <= GROUP_BYTES))
-                    j1++;
-                if (nn - j1 < GROUP_FEATS / 2) j1 = nn;  // no short last group
-                groups.push_back({j0, j1});
-                na = std::max(na, abase[j1] - abase[j0]);
-                nb = std::max(nb, bbase[j1] - bbase[j0]);
-                nt = std::max(nt, tbase[j1] - tbase[j0]);
-            }
+            const uint64_t na = plan.slots.a, nb = plan.slots.b, nt = plan.slots.t;
             SkEntry *A = s->alloc<SkEntry>(na * L, "sketch summaries");
             SkEntry *B = s->alloc<SkEntry>(nb * 2 * L, "sketch summaries");
             SkEntry *Tm = s->alloc<SkEntry>(nt * L, "sketch final merges");
@@ -1163,12 +1137,8 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
             const uint32_t cut_lds = 4 * (uint32_t)L + 4 * max_bin;
             sk_check(allow_lds(sk_cuts_kernel), "LDS attribute");
             sk_check(allow_lds(sk_merge_kernel), "LDS attribute");
-            // Room for every group's tables: at most a pruning merge a batch, and fewer
-            // final merges than slots for them.
-            uint8_t *tab = s->alloc<uint8_t>(sizeof(SkSortTask) * abase[nn] +
-                                                 sizeof(SkMergeTask) * (abase[nn] + tbase[nn]) +
-                                                 sizeof(SkCutTask) * (uint64_t)nn,
-                                             "sketch task tables");
+            // (room for every group's tables)
+            uint8_t *tab = s->alloc<uint8_t>(task_bytes(plan.slots, nn), "sketch task tables");
             std::vector<SkSortTask> sorts;
             std::vector<SkMergeTask> merges;
             std::vector<uint64_t> level_end;  // merges of levels 0..l end at level_end[l]
@@ -1176,7 +1146,7 @@ int fbh_sketch_cuts(fbh_sketch *s, float *cut_values, uint64_t values_capacity,
             std::vector<SkCutTask> cut_tasks;
             std::vector<uint8_t> host;
             // A group's tables are built and sent while the groups before it run.
-            for (const Group &g : groups) {
+            for (const SketchPlan::Group &g : plan.groups) {
                 sorts.clear();
                 merges.clear();
                 level_end.clear();

@@ -65,3 +65,44 @@ def test_a_failed_regrow_leaves_no_pointer(tmp_path):
     regrow(p, bytes, 32, release, take);
     CHECK(p == &blocks[1] && bytes == 64 && taken == 0);
     CHECK(freed.size() == 2 && freed[1] == nullptr);""")
+
+
+def test_sketch_bound_covers_every_layout(tmp_path):
+    """What the sketch's buffers are said to need covers the layout of any batch
+    counts: all features full, mixed with missing values, or empty."""
+    run_cpp(tmp_path, """
+    std::mt19937_64 r(7);
+    for (int it = 0; it < 4000; it++) {
+        const uint32_t n = 1 + r() % (it % 4 ? 700 : 5000);
+        const uint64_t limit = 16ull << r() % 11;
+        const uint64_t most = 1 + r() % (it % 3 ? 40 : 3000);
+        const uint32_t kind = it % 5;
+        std::vector<uint64_t> m(n);
+        for (auto &v : m)
+            v = kind == 0 ? most : kind == 1 ? r() % (most + 1) : kind == 2 ? r() % 2
+                : kind == 3 ? (r() % 2 ? most : 1) : (r() % 5 ? most : 0);
+        for (auto &v : m) v = std::min(v, most);
+        const SketchPlan p = sketch_plan(m, limit);
+        const SketchSlots b = sketch_slots_most(most, n, limit);
+        CHECK(p.slots.a <= b.a && p.slots.b <= b.b && p.slots.t <= b.t);
+        CHECK(p.slots.all_a <= b.all_a && p.slots.all_t <= b.all_t);
+        CHECK(p.groups.front().j0 == 0 && p.groups.back().j1 == n);
+        for (size_t g = 0; g + 1 < p.groups.size(); g++) {
+            CHECK(p.groups[g].j1 == p.groups[g + 1].j0);
+            CHECK(p.abase[p.groups[g].j1] - p.abase[p.groups[g].j0] <= p.slots.a);
+        }
+    }""")
+
+
+def test_sketch_bytes_count_the_groups_buffers():
+    """400k x 2000 at 256 bins: 11 GB of summaries in groups of features, not the 33
+    that all features' would take at once; and no less than the values alone."""
+    from ferrisboost_amd import _native as N
+
+    got = N.hip().fbh_sketch_device_bytes(400_000, 2000, 256, None)
+    assert 11e9 < got < 16e9
+    # few features share one group: every batch's entries, merged and final ones
+    m = -(-1_000_000 // 4096)
+    got = N.hip().fbh_sketch_device_bytes(1_000_000, 10, 256, None)
+    least = 4 * 1_000_000 * 10 + 10 * 16 * 4096 * (m + 2 * ((m + 1) // 2) + 1)
+    assert least < got < 2 * least
