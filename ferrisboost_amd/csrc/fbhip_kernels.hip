@@ -3522,8 +3522,12 @@ __global__ __launch_bounds__(PACK_ROWS_TPB) void pack_rows_kernel(
 #pragma unroll
         for (uint32_t k = 0; k < 8; k++) {
             const PackCellDev C = cells[L.first + min(c0 + k, L.count - 1)];
-            if (C.width == 1) mine[C.off] = (uint8_t)v[k];
-            else *reinterpret_cast<uint16_t *>(mine + C.off) = (uint16_t)v[k];
+            if (C.width == 1) {
+                mine[C.off] = (uint8_t)v[k];
+            } else {  // (a 16-bit layout's offsets are even; the words were cleared as such)
+                const uint16_t h = (uint16_t)v[k];
+                __builtin_memcpy(__builtin_assume_aligned(mine + C.off, 2), &h, 2);
+            }
         }
     }
     __syncthreads();
