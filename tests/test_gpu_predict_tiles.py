@@ -92,3 +92,36 @@ def test_large_and_few_trees(lib, rows, n_trees, depth, nf, n_cat, full):  # noq
     """Both sides of predict_tiles_pay, and of the row widths of the walk it leaves
     the others to."""
     test_margins_and_leaf_ids(lib, rows, n_trees, depth, nf, n_cat, full)
+
+
+@pytest.mark.parametrize("rows,n_trees,depth,nf,n_cat", [
+    (300, 40, 6, 28, 4),       # rows and trees in LDS
+    (20_000, 3, 12, 28, 4),    # nodes from memory, rows in LDS
+    (33_000, 2, 5, 400, 5),    # both from memory
+])
+def test_values_at_the_ends_of_the_order(lib, rows, n_trees, depth, nf, n_cat):  # noqa: F811
+    """Cells and thresholds among both zeros, infinities, denormals, the largest and
+    smallest numbers and NaN, equal ones among them: the walk's float comparisons."""
+    N = lib
+    rng = np.random.default_rng(nf + depth)
+    offs, a, words = _ensemble(rng, n_trees, depth, nf, n_cat, True)
+    tiny, big = np.float32(1.4e-45), np.finfo(np.float32).max
+    ends = np.array([0.0, -0.0, np.inf, -np.inf, tiny, -tiny, 3 * tiny, 1.17e-38, -1.17e-38, big,
+                     -big, 1.0, -1.0, np.nan], np.float32)
+    a["cond"] = rng.choice(ends, a["cond"].size).astype(np.float32)
+    x = rng.choice(ends, (rows, nf)).astype(np.float32)
+    h = C.c_void_p()
+    N.check_hip(N.hip().fbh_shap_model_create(
+        0, n_trees, N.ptr(offs), N.ptr(a["feat"]), N.ptr(a["cond"]), N.ptr(a["left"]),
+        N.ptr(a["right"]), N.ptr(a["dl"]), N.ptr(a["leaf"]), N.ptr(a["val"]), N.ptr(a["hess"]),
+        N.ptr(a["coff"]), N.ptr(a["clen"]), N.ptr(words), words.size, nf, 0.25, C.byref(h)))
+    try:
+        want, ids = _walk(offs, a, words, x)
+        got = np.full(rows, np.nan, np.float32)
+        N.check_hip(N.hip().fbh_predict(h, N.ptr(x), rows, None, 0, N.ptr(got)))
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        leaf = np.full((rows, n_trees), np.nan, np.float32)
+        N.check_hip(N.hip().fbh_predict(h, N.ptr(x), rows, None, 2, N.ptr(leaf)))
+        assert np.array_equal(leaf, ids)
+    finally:
+        N.hip().fbh_shap_model_destroy(h)

@@ -105,6 +105,40 @@ def test_paths_match_the_host_order(lib, rows, n_trees, depth, nf, n_cat, full):
         N.hip().fbh_shap_model_destroy(h)
 
 
+@pytest.mark.parametrize("nan_threshold", [False, True])
+def test_decisions_at_the_ends_of_the_order(lib, nan_threshold):
+    """Cells and thresholds among zeros, infinities, denormals and NaN: the lane masks'
+    decisions are the engine's (a NaN threshold takes its order whole). Tolerance as
+    above."""
+    N = lib
+    rng = np.random.default_rng(3)
+    rows, n_trees, nf = 200, 12, 9
+    offs, a, words = _ensemble(rng, n_trees, 6, nf, 2, True)
+    tiny, big = np.float32(1.4e-45), np.finfo(np.float32).max
+    ends = np.array([0.0, -0.0, np.inf, -np.inf, tiny, -tiny, 1.17e-38, big, -big, 1.0, np.nan],
+                    np.float32)
+    a["cond"] = rng.choice(ends[:-1], a["cond"].size).astype(np.float32)
+    if nan_threshold:
+        a["cond"][np.flatnonzero((a["leaf"] == 0) & (a["clen"] == 0))[0]] = np.nan
+    x = rng.choice(ends, (rows, nf)).astype(np.float32)
+    h = C.c_void_p()
+    N.check_hip(N.hip().fbh_shap_model_create(
+        0, n_trees, N.ptr(offs), N.ptr(a["feat"]), N.ptr(a["cond"]), N.ptr(a["left"]),
+        N.ptr(a["right"]), N.ptr(a["dl"]), N.ptr(a["leaf"]), N.ptr(a["val"]), N.ptr(a["hess"]),
+        N.ptr(a["coff"]), N.ptr(a["clen"]), N.ptr(words), words.size, nf, 0.25, C.byref(h)))
+    tol = 8 * 16 * 2.0 ** -24 * sum(float(np.abs(a["val"][b:e]).max())
+                                    for b, e in zip(offs[:-1], offs[1:]))
+    try:
+        out = {}
+        for order in (0, 1):
+            out[order] = np.full((rows, nf + 1), np.nan, np.float32)
+            N.check_hip(N.hip().fbh_shap_set_host_order(h, order))
+            N.check_hip(N.hip().fbh_shap_contribs(h, N.ptr(x), rows, None, N.ptr(out[order])))
+        assert np.max(np.abs(out[0] - out[1])) <= (0.0 if nan_threshold else tol)
+    finally:
+        N.hip().fbh_shap_model_destroy(h)
+
+
 @pytest.mark.parametrize("share,fits", [(1e-3, True), (1e-5, True), (1e-6, False)])
 def test_weights_near_the_range_of_a_float(lib, share, fits):
     """A path of eight splits on as many features that each pass `share` of the cover
