@@ -20,7 +20,8 @@ uint64_t keep_bytes(int device) noexcept;   // device memory kept
 bool drop_parked(int device) noexcept;      // destroys parked models (fbhip_shap.hip);
 uint64_t parked_bytes(int device) noexcept; // whether there were any; their memory
 hipError_t keep_stream(hipStream_t *s);     // a non-blocking stream
-hipError_t keep_stream_back(int device, hipStream_t s) noexcept;  // waits for it
+hipError_t keep_stream_back(int device, hipStream_t s, bool idle = false) noexcept;  // waits for
+                                                                                     // it if not idle
 
 constexpr int HIST_TPB = 256;      // threads of one histogram workgroup
 constexpr int SPLIT_TPB = 256;     // threads of one split-scan workgroup

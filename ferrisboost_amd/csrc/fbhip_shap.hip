@@ -782,6 +782,7 @@ struct fbh_shap_model {
     void *staging = nullptr, *pinned = nullptr;
     uint64_t staging_bytes = 0, array_bytes = 0;
     static constexpr uint64_t SMALL_WORK = 1 << 20;
+    bool in_flight = false;   // something may be: enqueued, and not waited for since
 
     ~fbh_shap_model() {
         if (device >= 0) (void)hipSetDevice(device);
@@ -794,7 +795,7 @@ struct fbh_shap_model {
     // the next one asks for again; `all` but what a few rows need (a block of
     // page-locked memory, a small workspace), which is not worth that.
     hipError_t rest(bool all) noexcept {
-        const hipError_t e = keep_stream_back(device, stream);
+        const hipError_t e = keep_stream_back(device, stream, !all && !in_flight);
         stream = nullptr;
         if (all || work_bytes > SMALL_WORK) {
             keep_free(KeepKind::device, work);
@@ -1240,6 +1241,7 @@ uint32_t pred_mode(Kind k) {
 void enqueue(fbh_shap_model *m, Kind k, const float *d_rows, uint64_t n, const float *d_margin,
              float *d_out) {
     if (n == 0) return;
+    m->in_flight = true;
     const uint32_t blocks = (uint32_t)((n + PRED_TPB - 1) / PRED_TPB);
     switch (k) {
         case Kind::Contribs:
@@ -1318,6 +1320,7 @@ void run_host(fbh_shap_model *m, Kind k, const Staging &st, const float *rows, u
         chk(hipMemcpyAsync(out + r0 * w, st.out, 4 * b * w, hipMemcpyDeviceToHost, m->stream),
             "output download");
         chk(hipStreamSynchronize(m->stream), "explain");
+        m->in_flight = false;
         float ms = 0.0f;
         chk(hipEventElapsedTime(&ms, m->e0, m->e1), "event");
         kernel_ms += ms;
@@ -1372,6 +1375,7 @@ void run_host_alloc(fbh_shap_model *m, Kind k, const float *rows, uint64_t n_row
         enqueue(m, k, x, n_rows, margin ? mg : nullptr, o);
         chk(hipEventRecord(m->e1, m->stream), "event");
         chk(hipStreamSynchronize(m->stream), "explain");
+        m->in_flight = false;
         std::memcpy(out, o, 4 * n_rows * w);
         float ms = 0.0f;
         chk(hipEventElapsedTime(&ms, m->e0, m->e1), "event");
