@@ -48,25 +48,29 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBPS = 8000.0
-# VALU issue peak: 256 CUs x 64 lanes x 2.4 GHz, one fp32 operation a lane a cycle (the
-# kernels are built without FMA contraction and without packed fp32).
+# VALU issue peak: 256 CUs x 64 lanes x 2.4 GHz, one instruction a lane a cycle (a fused
+# multiply-add is one; the kernels are built without packed fp32).
 VALU_PEAK_TOPS = 39.3
-# TreeSHAP of the 100-tree depth-8 ensemble: VALU lane-operations a row, counted by
-# SQ_INSTS_VALU x 64 / rows for shap_rec_kernel on the shap workload.
-SHAP_VALU_OPS_PER_ROW = 11.23e6
-# Prediction of the same ensemble: VALU lane-operations a row (SQ_INSTS_VALU x 64 / rows
-# for predict_lds4_kernel on the predict workload).
-PREDICT_VALU_OPS_PER_ROW = 11934
+# VALU lane-operations a row (SQ_INSTS_VALU x 64 / rows) of the 100-tree depth-8 ensemble,
+# counted on the workloads themselves (profiles/shap_kernel.md, predict_kernel.md):
+# shap_masks_kernel, shap_paths_kernel and shap_paths_sum_kernel; predict_tile_kernel.
+SHAP_VALU_OPS_PER_ROW = 1.344e6
+PREDICT_VALU_OPS_PER_ROW = 16290
 # MI355X fp32 vector peak (FMA counted as two operations).
 FP32_PEAK_TFLOPS = 157.3
-# QuadratureTreeSHAP's arithmetic (8 quadrature points): for each child edge of an
-# internal node the extend (3 operations a point) and the unwind of that edge's
-# contribution (5 a point), plus the sum of the two subtrees' returns (1 a point); for a
-# leaf the scaled return (2 a point, and the path weight). The unwinds of a feature met
-# twice on a path are data-dependent and not counted: a lower bound.
-SHAP_QP = 8
-SHAP_FLOPS_INTERNAL = 2 * (3 + 5) * SHAP_QP + SHAP_QP
-SHAP_FLOPS_LEAF = 2 * SHAP_QP + 1
+# TreeSHAP's arithmetic as closed sums over a node's two children at 4 quadrature points
+# (fbhip_shap_paths.hip), an FMA counted as two: for each split child the factors above it
+# (3 operations a point), its sum into the node's (1) and its contribution (2); for a node
+# with a split child its own sum and contribution (4 a point) and what its leaf children
+# give (3); for a node of two leaves those (3), its sums (2 a point) and its contribution
+# (4). Features met twice on a path are data-dependent and not counted: a lower bound.
+SHAP_POINTS = 4
+
+
+def shap_flops_per_node(split_children: int) -> int:
+    if split_children == 0:
+        return 3 + 2 * SHAP_POINTS + 4
+    return 6 * SHAP_POINTS * split_children + 4 * SHAP_POINTS + 3
 
 
 def shap_flops_per_row(model) -> int:
@@ -74,8 +78,11 @@ def shap_flops_per_row(model) -> int:
     model (the same for every row: every row visits every node)."""
     total = 0
     for t in model.trees():
-        leaves = int((t["is_leaf"] == 1).sum())
-        total += SHAP_FLOPS_INTERNAL * (t.size - leaves) + SHAP_FLOPS_LEAF * leaves
+        inner = np.flatnonzero(t["is_leaf"] != 1)
+        split = (t["is_leaf"][t["left"][inner]] != 1).astype(int) + (
+            t["is_leaf"][t["right"][inner]] != 1)
+        for k in range(3):
+            total += shap_flops_per_node(k) * int((split == k).sum())
     return total
 
 
@@ -431,9 +438,9 @@ def predict_workload(args):
               "trees": 100, "max_depth": 8}
     out = base_line(args, round(rows_per_s, 1), "rows/s", round(kernel_ms / args.steps, 3),
                     config, dtype="f32")
-    # The walk is a chain of dependent loads (node, then the row's cell, then
-    # the child), so its bound is memory latency, not bandwidth or VALU
-    # issue: the VALU and HBM figures beside it are far from their peaks.
+    # The walk is a chain of dependent LDS reads (node, then the row's cell, then
+    # the child), so its bound is their latency, not bandwidth or VALU issue:
+    # the VALU and HBM figures beside it are far from their peaks.
     valu = rows_per_s * PREDICT_VALU_OPS_PER_ROW / 1e12
     out.update({
         "roofline": {"bound": "latency", "achieved": round(rows_per_s * visits / 1e9, 2),
@@ -492,7 +499,9 @@ def shap_workload(args):
     out = base_line(args, round(rows_per_s, 1), "rows/s", round(kernel_ms / args.steps, 3),
                     config, dtype="f32")
     out.update({
-        "roofline": {"bound": "valu", "achieved": round(tops, 2), "peak": VALU_PEAK_TOPS,
+        # (a wave's sums take most of a CU's LDS, so three waves a CU wait for each other's
+        # chains of multiply-adds: the issue rate below is far from its peak)
+        "roofline": {"bound": "latency", "achieved": round(tops, 2), "peak": VALU_PEAK_TOPS,
                      "unit": "T lane-ops/s", "frac": round(tops / VALU_PEAK_TOPS, 4),
                      "traffic": None, "ops_per_row": SHAP_VALU_OPS_PER_ROW,
                      "algorithmic_flops_per_row": alg,
