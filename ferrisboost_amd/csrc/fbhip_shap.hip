@@ -34,6 +34,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <vector>
 
 using namespace fbh;
@@ -1721,8 +1722,14 @@ int fbh_shap_model_create(int device, uint32_t n_trees, const uint32_t *tree_off
         // on one thread, 2.9 without the others; 100 trees 1.5, 1.3 and 1.0.
         constexpr uint32_t THREADS_LEAST = 1 << 16;  // nodes
         if (total >= THREADS_LEAST) {
-            auto paths = std::async(std::launch::async, make_paths);
-            auto runs = std::async(std::launch::async, make_runs);
+            auto start = [](auto &f) {
+                try {
+                    return std::async(std::launch::async, std::ref(f));
+                } catch (const std::system_error &) {  // no thread to be had: made by get()
+                    return std::async(std::launch::deferred, std::ref(f));
+                }
+            };
+            auto paths = start(make_paths), runs = start(make_runs);
             m->upload(arrays);
             arrays = {};
             paths.get();

@@ -48,6 +48,7 @@
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <vector>
@@ -831,9 +832,13 @@ struct RowPipe {
             }
             failed[t] = e;
         };
-        std::thread other(work, 1);
+        std::thread other;
+        try {
+            other = std::thread(work, 1);
+        } catch (const std::system_error &) {  // no thread to be had: one copies all pieces
+        }
         work(0);
-        other.join();
+        if (other.joinable()) other.join();
         for (hipError_t e : failed) sk_check(e, "row upload");
     }
     // Once nothing of it is in flight.

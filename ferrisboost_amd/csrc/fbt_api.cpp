@@ -8,6 +8,7 @@
 #include <limits>
 #include <memory>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <utility>
 
@@ -372,7 +373,12 @@ public:
         }
         for (uint64_t i = 0; i < k; i++) {
             const uint64_t b = n * i / k, e = n * (i + 1) / k;
-            parts_.push_back(std::async(std::launch::async, [=] { return holds_reserved(x + b, e - b); }));
+            const auto part = [=] { return holds_reserved(x + b, e - b); };
+            try {
+                parts_.push_back(std::async(std::launch::async, part));
+            } catch (const std::system_error &) {  // no thread to be had: looked through by check()
+                parts_.push_back(std::async(std::launch::deferred, part));
+            }
         }
     }
     void check() {
