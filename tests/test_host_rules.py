@@ -106,3 +106,17 @@ def test_sketch_bytes_count_the_groups_buffers():
     got = N.hip().fbh_sketch_device_bytes(1_000_000, 10, 256, None)
     least = 4 * 1_000_000 * 10 + 10 * 16 * 4096 * (m + 2 * ((m + 1) // 2) + 1)
     assert least < got < 2 * least
+
+
+def test_the_integration_recipe_builds_every_source():
+    """INTEGRATION.md's build step names the sources of the library, with the flags that
+    its results depend on."""
+    import re
+
+    from ferrisboost_amd import build
+
+    with open(os.path.join(os.path.dirname(os.path.dirname(CSRC)), "INTEGRATION.md")) as f:
+        recipe = re.search(r"// build.rs.*?```", f.read(), flags=re.S).group(0)
+    assert sorted(re.findall(r"\{src\}/(\w+\.hip)", recipe)) == sorted(build.BACKEND_SRCS)
+    flags = [f for f in build.HIP_FLAGS if not f.startswith("-W")]
+    assert all(f'"{f}"' in recipe for f in flags)
