@@ -1339,12 +1339,12 @@ constexpr uint64_t PINNED_BYTES = 256ull << 10;
 uint64_t round256(uint64_t v) { return (v + 255) & ~uint64_t(255); }
 
 // Whether the kind's kernels read a row a few times in order and write each output
-// once, and fetch them faster than two copies would bring them. The workgroup that
-// copies 64 rows for contributions waits for them row by row: 64 x 28 (15 KB in and
-// out, 20 trees of depth 5) 80 us in place, 81 with copies, 64 x 50 (26 KB) 79 and 93,
-// 8 x 500 (32 KB) 89 and 90, 64 x 100 (52 KB) 101 and 90, 64 x 500 239 and 148.
-// Predictions' 1024 threads have theirs under way at once: 64 x 500 48 and 56.
-constexpr uint64_t IN_PLACE_TILE_BYTES = 32 << 10;
+// once, and fetch them faster than two copies would bring them. Contributions (one
+// workgroup copies 64 rows; 20 trees of depth 5): 64 x 28 (15 KB in and out) 61 us in
+// place, 82 with copies, 64 x 100 (52 KB) 71 and 80, 64 x 200 (103 KB) 88 and 92,
+// 32 x 500 (128 KB) 97 and 100, 64 x 500 (257 KB) 127 and 120. Predictions' 1024
+// threads have more under way: 64 x 500 48 and 56.
+constexpr uint64_t IN_PLACE_TILE_BYTES = 160 << 10;
 bool runs_in_place(const fbh_shap_model *m, Kind k, uint64_t n) {
     if (k == Kind::Contribs)
         return takes_paths(m, false) &&

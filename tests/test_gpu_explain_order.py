@@ -86,15 +86,16 @@ def test_the_order_applies_to_treeshap_alone(models):
             m.predict(x, engine_order=True, **kw)
 
 
-@pytest.mark.parametrize("nf,rows", [(63, 63), (63, 64), (64, 65), (511, 8), (512, 8), (300, 9)])
+@pytest.mark.parametrize("nf,rows", [(1, 3), (63, 64), (64, 65), (255, 64), (256, 9), (319, 64),
+                                     (320, 64), (500, 40), (500, 41)])
 def test_wide_rows_on_both_sides_of_the_copies(nf, rows):
-    """Contributions of rows read over the link and of rows copied first (32 KiB of 64
+    """Contributions of rows read over the link and of rows copied first (160 KiB of 64
     rows in and out is where they part): the same bits as in a batch of 700."""
     import ferrisboost_amd as fb
 
     rng = np.random.default_rng(nf)
     x = rng.normal(size=(ROWS, nf)).astype(np.float32)
-    m = fb.train({"max_depth": 4, "objective": "reg:squarederror"}, x, x[:, 0] * x[:, 1],
+    m = fb.train({"max_depth": 4, "objective": "reg:squarederror"}, x, x[:, 0] * x[:, -1],
                  num_boost_round=5)
     whole = m.predict(x, pred_contribs=True)
     part = m.predict(x[:rows], pred_contribs=True)
