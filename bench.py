@@ -54,7 +54,7 @@ VALU_PEAK_TOPS = 39.3
 # VALU lane-operations a row (SQ_INSTS_VALU x 64 / rows) of the 100-tree depth-8 ensemble,
 # counted on the workloads themselves (profiles/shap_kernel.md, predict_kernel.md):
 # shap_masks_kernel, shap_paths_kernel and shap_paths_sum_kernel; predict_tile_kernel.
-SHAP_VALU_OPS_PER_ROW = 1.344e6
+SHAP_VALU_OPS_PER_ROW = 1.347e6
 PREDICT_VALU_OPS_PER_ROW = 16290
 # MI355X fp32 vector peak (FMA counted as two operations).
 FP32_PEAK_TFLOPS = 157.3
